@@ -338,7 +338,7 @@ __device__ inline bool emit(const Args &a, long long gi, Photon &p, Acc &acc) {
     const bool emits = bn > 1.0f;
     const float s2 = emits ? 1.0f - 1.0f / (bn * bn) : 0.0f;
     p.w0 = TWO_PI * FINE_STRUCTURE * S.charge * S.charge * S.length * s2 * zq * 1e9f * S.weight;
-    const float cos_c = emits ? 1.0f / bn : 1.0f;
+    const float cos_c = emits ? div_ieee(1.0f, bn) : 1.0f;
     const float sin_c = sqrtf(fmaxf(1.0f - cos_c * cos_c, 0.0f));
     float sp, cp;
     __sincosf(TWO_PI * u[2], &sp, &cp);
@@ -596,7 +596,7 @@ __device__ inline float deposit_cotangent(const Args &a, const AdjArgs *b, const
   return (float)cw;
 }
 
-__device__ __forceinline__ float ratio(float live, float ref) { return ref != 0.0f ? live / ref : 0.0f; }
+__device__ __forceinline__ float ratio(float live, float ref) { return ref != 0.0f ? div_ieee(live, ref) : 0.0f; }
 
 // ------------------------------------------------------------------------------------------- the diffusion jump
 // At a Rayleigh event in a medium with a clearance grid, with a linear polarisation (ei = 0): the photon walks its
@@ -789,7 +789,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
         if (((support >> k) & 1) && !(sr.p[k] > 0.0f)) pdraw[k] = eps;
     }
     for (int k = 0; k < N_OUT; ++k) tot += pdraw[k];
-    for (int k = 0; k < N_OUT; ++k) pprop[k] = tot > 0.0f ? pdraw[k] / tot : 0.0f;
+    for (int k = 0; k < N_OUT; ++k) pprop[k] = tot > 0.0f ? div_ieee(pdraw[k], tot) : 0.0f;
     o = choose6(pprop, u[2]);
     // the deposit: the expected detection at the crossing (step.py:522-524)
     const float dep_q = p.w * reach_live * att * sl.detect;

@@ -247,18 +247,46 @@ __device__ inline void torus_intervals(float R, float r, float3 w, float3 y, flo
   if (nr >= 4) { a1 = tc + r2; b1 = tc + r3; }
 }
 
-// a leaf's (at most two) intervals [lo, hi) along o + t d in its kind's frame; face 0 the quadric, k + 1 plane k.
-// TOR: the scene has torus leaves (a kernel feature: the root isolation costs registers every other kernel keeps)
-template <bool TOR>
-__device__ inline void leaf_intervals(const Geo &g, int li, float3 o, float3 d, LeafIv &iv) {
-  const float4 L0 = g.leaf[4 * li], L1 = g.leaf[4 * li + 1], L2 = g.leaf[4 * li + 2], L3 = g.leaf[4 * li + 3];
-  const int typ = __float_as_int(L3.y), p0 = __float_as_int(L3.z), np = __float_as_int(L3.w);
+// a leaf's four records: (q, c), (A00 A01 A02 A11), (A12 A22 b0 b1), (b2, typ, p0, np)
+struct LeafRec {
+  float4 L0, L1, L2, L3;
+};
+
+__device__ __forceinline__ LeafRec leaf_rec(const Geo &g, int li) {
+  return LeafRec{g.leaf[4 * li], g.leaf[4 * li + 1], g.leaf[4 * li + 2], g.leaf[4 * li + 3]};
+}
+
+// a / b by one reciprocal and one product: the compiler's approximate quotient without its scaling of denominators
+// beyond 2^96, which no length, slope or index here comes near (a rounded product: never fused into a sum after it)
+__device__ __forceinline__ float div_fast(float a, float b) {
+#pragma clang fp contract(off)
+  return a * __builtin_amdgcn_rcpf(b);
+}
+
+// the correctly rounded quotient, where the source asks for it and not where the optimiser moves a division to: the
+// hardware's scaled Newton steps, the residual of the quotient applied twice
+__device__ __forceinline__ float div_ieee(float a, float b) {
+  bool sn, sd;
+  const float n = __builtin_amdgcn_div_scalef(a, b, true, &sn), d = __builtin_amdgcn_div_scalef(a, b, false, &sd);
+  const float r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+  float q = n * r;
+  q = fmaf(fmaf(-d, q, n), r, q);
+  return __builtin_amdgcn_div_fixupf(__builtin_amdgcn_div_fmasf(fmaf(-d, q, n), r, q, sn), b, a);
+}
+
+// a leaf's (at most two) intervals [lo, hi) along o + t d in its kind's frame; face 0 the quadric, k + 1 plane k, read
+// by plane(k).  TOR: the scene has torus leaves (a kernel feature: the root isolation costs registers every other
+// kernel keeps)
+template <bool TOR, class PL>
+__device__ inline void leaf_intervals_of(const LeafRec &r, PL plane, float3 o, float3 d, LeafIv &iv) {
+  const float4 L0 = r.L0, L1 = r.L1, L2 = r.L2, L3 = r.L3;
+  const int typ = __float_as_int(L3.y), np = __float_as_int(L3.w);
   const float3 y = sub3(o, mk3(L0.x, L0.y, L0.z));
   float tp0 = -HUGEF, tp1 = HUGEF;
   int fp0 = -1, fp1 = -1;
   bool empty = false;
   for (int k = 0; k < np; ++k) {
-    const float4 P = g.plane[p0 + k];
+    const float4 P = plane(k);
     const float nd = P.x * d.x + P.y * d.y + P.z * d.z;
     const float rhs = P.w - (P.x * y.x + P.y * y.y + P.z * y.z);
     if (fabsf(nd) < 1e-12f) {
@@ -319,7 +347,7 @@ __device__ inline void leaf_intervals(const Geo &g, int li, float3 o, float3 d, 
       } else {
         const float sq = sqrtf(D);
         const float qq = -(beta + copysignf(sq, beta));
-        float r1 = qq / a, r2 = qq != 0.0f ? gam / qq : r1;
+        float r1 = div_fast(qq, a), r2 = qq != 0.0f ? div_ieee(gam, qq) : r1;
         const float rl = fminf(r1, r2), rh = fmaxf(r1, r2);
         if (a > 0.0f) {
           a0 = tc + rl; b0 = tc + rh; qa0 = qb0 = true;
@@ -347,6 +375,13 @@ __device__ inline void leaf_intervals(const Geo &g, int li, float3 o, float3 d, 
     iv.flo[1] = (a1 > tp0 && qa1) ? 0 : fp0;
     iv.fhi[1] = (b1 < tp1 && qb1) ? 0 : fp1;
   }
+}
+
+template <bool TOR>
+__device__ __forceinline__ void leaf_intervals(const Geo &g, int li, float3 o, float3 d, LeafIv &iv) {
+  const LeafRec r = leaf_rec(g, li);
+  const float4 *pl = g.plane + __float_as_int(r.L3.z);
+  leaf_intervals_of<TOR>(r, [&](int k) { return pl[k]; }, o, d, iv);
 }
 
 // a leaf's membership of a point (its kind's frame)
@@ -408,11 +443,10 @@ struct Change {
   float3 n;        // the face's normal there, in the solid's frame (not normalised)
 };
 
-// the normal of leaf li's face `face` (0 the quadric: A y + b at y = o + t d - q; k >= 1 plane k) in its frame; the
-// leaf's data was just read by its interval test, so these reads hit the cache
-template <bool TOR>
-__device__ __forceinline__ float3 leaf_normal(const Geo &g, int li, int face, float3 o, float3 d, float t) {
-  const float4 L0 = g.leaf[4 * li], L1 = g.leaf[4 * li + 1], L2 = g.leaf[4 * li + 2], L3 = g.leaf[4 * li + 3];
+// the normal of a leaf's face `face` (0 the quadric: A y + b at y = o + t d - q; k >= 1 plane k) in its frame
+template <bool TOR, class PL>
+__device__ __forceinline__ float3 leaf_normal_of(const LeafRec &r, PL plane, int face, float3 o, float3 d, float t) {
+  const float4 L0 = r.L0, L1 = r.L1, L2 = r.L2, L3 = r.L3;
   if (face == 0) {
     const float3 y = sub3(fma3(t, d, o), mk3(L0.x, L0.y, L0.z));
     if (TOR && __float_as_int(L3.y) == 2) {  // a torus: y - R (the point's direction across the axis)
@@ -424,10 +458,42 @@ __device__ __forceinline__ float3 leaf_normal(const Geo &g, int li, int face, fl
     return mk3(L1.x * y.x + L1.y * y.y + L1.z * y.z + L2.z, L1.y * y.x + L1.w * y.y + L2.x * y.z + L2.w,
                L1.z * y.x + L2.x * y.y + L2.y * y.z + L3.x);
   }
-  const float4 P = g.plane[__float_as_int(L3.z) + face - 1];
+  const float4 P = plane(face - 1);
   return mk3(P.x, P.y, P.z);
 }
 
+// ... of leaf li (its data was just read by its interval test, so these reads hit the cache)
+template <bool TOR>
+__device__ __forceinline__ float3 leaf_normal(const Geo &g, int li, int face, float3 o, float3 d, float t) {
+  const LeafRec r = leaf_rec(g, li);
+  const float4 *pl = g.plane + __float_as_int(r.L3.z);
+  return leaf_normal_of<TOR>(r, [&](int k) { return pl[k]; }, face, o, d, t);
+}
+
+// first_change for a solid of one leaf: its intervals are the solid's
+template <bool TOR, class PL>
+__device__ inline Change first_change_one(const LeafRec &r, PL plane, int vol, float3 o, float3 d, bool exit_query,
+                                          int skip_code, float skip_t) {
+  Change ch{HUGEF, -1, -1, mk3(0.f, 0.f, 1.f)};
+  LeafIv iv;
+  leaf_intervals_of<TOR>(r, plane, o, d, iv);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    float lo = iv.lo[p], hi = iv.hi[p];
+    if (lo >= HUGEF) continue;
+    if (srf_code(vol, 0, iv.flo[p]) == skip_code && fabsf(lo) <= skip_t) lo = -BIGF;
+    if (srf_code(vol, 0, iv.fhi[p]) == skip_code && fabsf(hi) <= skip_t) hi = -BIGF;
+    if (exit_query) {
+      if (lo <= 0.0f && 0.0f < hi && hi < ch.t) { ch.t = hi; ch.leaf = 0; ch.face = iv.fhi[p]; }
+    } else {
+      if (lo > 0.0f && lo < hi && lo < ch.t) { ch.t = lo; ch.leaf = 0; ch.face = iv.flo[p]; }
+    }
+  }
+  if (exit_query && ch.leaf < 0)  // the start is outside its own solid (rounding): leave it where it is, the
+    return Change{0.0f, 0, 0, mul3(-1.0f, d)};  // normal facing the photon (no face is met)
+  if (ch.leaf >= 0) ch.n = leaf_normal_of<TOR>(r, plane, ch.face, o, d, ch.t);
+  return ch;
+}
 
 // the first change of the solid's membership along the ray after t = 0, from the side `want_from` (true: the
 // point starts inside and the change is an exit; false: an entry).  Endpoints on the face `skip_code` within
@@ -436,25 +502,10 @@ template <bool TOR>
 __device__ inline Change first_change(const Geo &g, int4 K, int vol, float3 o, float3 d, bool exit_query,
                                       int skip_code, float skip_t) {
   Change ch{HUGEF, -1, -1, mk3(0.f, 0.f, 1.f)};
-  if (K.y == 1) {  // one leaf: its intervals are the solid's
-    LeafIv iv;
-    leaf_intervals<TOR>(g, K.x, o, d, iv);
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      float lo = iv.lo[p], hi = iv.hi[p];
-      if (lo >= HUGEF) continue;
-      if (srf_code(vol, 0, iv.flo[p]) == skip_code && fabsf(lo) <= skip_t) lo = -BIGF;
-      if (srf_code(vol, 0, iv.fhi[p]) == skip_code && fabsf(hi) <= skip_t) hi = -BIGF;
-      if (exit_query) {
-        if (lo <= 0.0f && 0.0f < hi && hi < ch.t) { ch.t = hi; ch.leaf = 0; ch.face = iv.fhi[p]; }
-      } else {
-        if (lo > 0.0f && lo < hi && lo < ch.t) { ch.t = lo; ch.leaf = 0; ch.face = iv.flo[p]; }
-      }
-    }
-    if (exit_query && ch.leaf < 0)  // the start is outside its own solid (rounding): leave it where it is, the
-      return Change{0.0f, 0, 0, mul3(-1.0f, d)};  // normal facing the photon (no face is met)
-    if (ch.leaf >= 0) ch.n = leaf_normal<TOR>(g, K.x, ch.face, o, d, ch.t);
-    return ch;
+  if (K.y == 1) {
+    const LeafRec r = leaf_rec(g, K.x);
+    const float4 *pl = g.plane + __float_as_int(r.L3.z);
+    return first_change_one<TOR>(r, [&](int k) { return pl[k]; }, vol, o, d, exit_query, skip_code, skip_t);
   }
   // several leaves: scan the endpoints in order for the first change of the program's value
   const int nl = K.y < MAX_CSG_LEAVES ? K.y : MAX_CSG_LEAVES;
@@ -541,7 +592,7 @@ __device__ inline void core_interval(const Geo &g, int vol, float3 xl, float3 dl
     const float disc = b * b - a * c;
     if (a > 0.0f && disc > 0.0f) {
       const float q = -(b + copysignf(sqrtf(disc), b));
-      const float r0 = q / a, r1 = q != 0.0f ? c / q : r0;
+      const float r0 = q / a, r1 = q != 0.0f ? div_ieee(c, q) : r0;
       t0 = fmaxf(t0, fminf(r0, r1));
       t1 = fminf(t1, fmaxf(r0, r1));
     } else if (!(a == 0.0f && c <= 0.0f)) {  // misses the cylinder (or runs along it outside)
