@@ -14,7 +14,7 @@ import json
 import os
 import time
 
-CHUNKS = (64, 128, 256, 512, 1024, 4096)
+CHUNKS = (0, 64, 128, 256, 512, 1024, 4096)  # 0: the engine's own split of the photons
 # the persistent grid's resident workgroups per CU: each photon-loop kernel's 768-thread workgroup of 12 wavefronts
 # fills a CU at its register budget, so "as many as fit" (0) is one and the search has nothing else to try
 BLOCKS = (0,)
@@ -49,7 +49,7 @@ def _key(run, what):
     return f"{run.det.name}|{what}|photons={run.total}|sources={len(run.rows)}|{name}"
 
 
-ADJ_CHUNKS = (128, 512, 2048)  # the adjoint's launches cost ~4 forward ones: a coarser grid, timed once each
+ADJ_CHUNKS = (0, 128, 512, 2048)  # the adjoint's launches cost ~4 forward ones: a coarser grid, timed once each
 
 
 def tune(run, what="forward", chunks=None, blocks=BLOCKS, repeats=None):

@@ -8,8 +8,9 @@
 // `arrival`, q w0 t to `arrival_t`, q w0 hat_k(lam) to `charge` and, when its photon ends, each sensor's square of
 // the photon's summed deposits to `arrival2` (the per-photon second moment).
 //
-// Schedule: each wavefront keeps 64 photons in flight; a lane whose photon ended takes the next one from a chunk its
-// wavefront claimed from the device work queue (one atomic per chunk), so lanes refill every step (the reference's
+// Schedule: each wavefront keeps 64 photons in flight; a lane whose photon ended takes the next one from its
+// wavefront's range, a first one of its own and then chunks claimed from the device work queue (one atomic per chunk),
+// so lanes refill every step (the reference's
 // "step" schedule, src/lumen/run.py:81) and a launch of many sources with uneven photon counts keeps every lane busy.
 #include <hip/hip_runtime.h>
 
@@ -56,7 +57,6 @@ template <unsigned F>
 constexpr int block_of() { return BLOCK; }
 template <unsigned F>
 constexpr int adj_block_of() { return BLOCK; }
-constexpr int DEFAULT_CHUNK = 256;
 constexpr int MAX_GRAD = 8192;  // gradient slots a block accumulates in LDS (64 KiB)
 constexpr long long LDS_TALLY_CELLS = 20480;  // tallies of at most this many cells (160 KiB) may go to LDS
 constexpr int OCC_CACHE = 8;
@@ -88,6 +88,8 @@ struct Args {
   uint32_t k0, k1;
   float roulette, max_dist, reach;
   int max_vert, chunk;
+  long long first_chunk;  // the photons of each wavefront's first range, its own by its index (claim_schedule)
+  long long dyn_at;       // where the first ranges end: the work queue hands out the photons past it, chunk by chunk
   int keep_zero;  // 1: a photon whose live weight became 0 walks on (the reference's records); 0: it ends
   int reach_on;   // 1: the reach bound where the model has one (the controls' reach_bound)
   double *__restrict__ tally;
@@ -146,6 +148,7 @@ struct Acc {  // per-lane health accumulators of the frequent fates, flushed onc
 // held all launch long for them would crowd the step's working set
 enum { RF_LOST = 0, RF_ESC, RF_DCUT, RF_ABAND, RF_TRUNC, RF_PUSHED, RF_SPILLS, RF_N };
 __shared__ float s_rare[RF_N];
+__shared__ double s_health[LH_HEALTH_N];  // the block's sums of its wavefronts' Acc (flush_health)
 // per wavefront of the block, the volume its last located emission started in: a new photon whose start lies in that
 // volume's daughter-free core starts in that volume (no daughter holds a point of the core), with no descent from the
 // top (-1: none yet; lanes overwrite it as they like, any value is only a hint that the core test checks)
@@ -1048,7 +1051,9 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// every thread of the block calls it (a barrier inside)
+// every thread of the block calls it (barriers inside): the wavefronts' sums meet in the block's LDS cells, and one
+// instruction adds the block's to the launch's.  Atomics on the one cache line of `health` take about 12 ns each: a
+// wavefront adding its own cells one by one (3,072 wavefronts, 8 cells) spent up to 250 us of a launch in line there
 __device__ inline void flush_health(const Args &a, const Acc &acc) {
   const float vals[LH_HEALTH_N] = {acc.bulk, acc.surf, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, acc.rou, acc.rew, 0.0f,
                                    (float)acc.records, 0.0f, (float)acc.vertices, (float)acc.photons, acc.start_w,
@@ -1057,19 +1062,28 @@ __device__ inline void flush_health(const Args &a, const Acc &acc) {
 #pragma unroll
   for (int k = 0; k < LH_HEALTH_N; ++k) {
     if (k == LH_H_LOST || k == LH_H_ESCAPED || k == LH_H_DISTANCE_CUT || k == LH_H_ABANDONED ||
-        k == LH_H_TRUNCATED || k == LH_H_PUSHED || k == LH_H_MOMENT_SPILLS || k == 15)
+        k == LH_H_TRUNCATED || k == LH_H_PUSHED || k == LH_H_MOMENT_SPILLS || k == LH_H_BOUNDED)
       continue;
     const float s = wave_sum(vals[k]);
-    if (lane == 0 && s != 0.0f) unsafeAtomicAdd(a.health + k, (double)s);
+    if (lane == 0 && s != 0.0f) atomicAdd(&s_health[k], (double)s);
   }
   __syncthreads();
-  if (threadIdx.x < RF_N) {
-    const int cell[RF_N] = {LH_H_LOST, LH_H_ESCAPED, LH_H_DISTANCE_CUT, LH_H_ABANDONED, LH_H_TRUNCATED, LH_H_PUSHED,
+  if (threadIdx.x < LH_HEALTH_N) {
+    const int rare[RF_N] = {LH_H_LOST, LH_H_ESCAPED, LH_H_DISTANCE_CUT, LH_H_ABANDONED, LH_H_TRUNCATED, LH_H_PUSHED,
                             LH_H_MOMENT_SPILLS};
-    const float v = s_rare[threadIdx.x];
-    if (v != 0.0f) unsafeAtomicAdd(a.health + cell[threadIdx.x], (double)v);
+    double v = s_health[threadIdx.x];
+    for (int k = 0; k < RF_N; ++k) v = (int)threadIdx.x == rare[k] ? (double)s_rare[k] : v;
+    if (threadIdx.x == LH_H_BOUNDED) v = (double)s_bounded;
+    if (v != 0.0) unsafeAtomicAdd(a.health + threadIdx.x, v);
   }
-  if (threadIdx.x == RF_N && s_bounded != 0u) unsafeAtomicAdd(a.health + LH_H_BOUNDED, (double)s_bounded);
+}
+
+// the block's own cells (s_rare, s_health, s_bounded, s_hint) at its start
+__device__ __forceinline__ void clear_block_cells() {
+  if (threadIdx.x == 0) s_bounded = 0u;
+  if (threadIdx.x < RF_N) s_rare[threadIdx.x] = 0.0f;
+  if (threadIdx.x < LH_HEALTH_N) s_health[threadIdx.x] = 0.0;
+  if (threadIdx.x < 32) s_hint[threadIdx.x] = -1;
 }
 
 __global__ void reset_queue(unsigned long long *q) { *q = 0ull; }
@@ -1138,13 +1152,42 @@ __device__ inline Args stage_tables(const Args &a0) {
   return a;
 }
 
+// A wavefront's range of the launch's photons.  Its first is its own by its index, wavefront w of every block before
+// wavefront w + 1 of any (a launch of few photons spreads over the CUs), so a launch begins without a claim: the
+// atomics on one address take 12 ns each, 37 us for the 3,072 wavefronts' first claims.  Past the first ranges the
+// wavefront claims chunks from the work queue; a launch whose first ranges hold every photon never touches it.
+struct Range {
+  long long cursor, end;
+  bool drained;
+};
+
+__device__ __forceinline__ Range first_range(const Args &a) {
+  const long long w = (long long)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+  const long long b = min(w * a.first_chunk, a.dyn_at);
+  return Range{b, min(b + a.first_chunk, a.dyn_at), false};
+}
+
+// the next chunk when the range is used up: false once there is none
+__device__ __forceinline__ bool next_range(const Args &a, Range &r, int lane) {
+  if (a.dyn_at < a.total) {
+    unsigned long long c = 0;
+    if (lane == 0) c = atomicAdd(a.queue, (unsigned long long)a.chunk);
+    const long long base = a.dyn_at + (long long)__shfl(c, 0);
+    if (base < a.total) {
+      r.cursor = base;
+      r.end = min(base + a.chunk, a.total);
+      return true;
+    }
+  }
+  r.drained = true;
+  return false;
+}
+
 template <unsigned F>
 __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args a0, int n_lds) {
   if (a0.lds_tally)
     for (int i = threadIdx.x; i < n_lds; i += blockDim.x) lds_cells[i] = 0.0;
-  if (threadIdx.x == 0) s_bounded = 0u;
-  if (threadIdx.x < RF_N) s_rare[threadIdx.x] = 0.0f;
-  if (threadIdx.x < 32) s_hint[threadIdx.x] = -1;
+  clear_block_cells();
   stage_nodes(a0.g);
   const Args a = stage_tables<F>(a0);
   __syncthreads();
@@ -1152,34 +1195,25 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
   Acc acc{};
   bool alive = false;
   const int lane = threadIdx.x & 63;
-  long long cursor = 0, chunk_end = 0;
-  bool drained = false;
+  Range r = first_range(a);
   for (;;) {
     // refill the lanes whose photon ended from the wavefront's chunk of the work queue
     bool need = !alive;
     unsigned long long mask = __ballot(need);
-    while (mask != 0ull && !drained) {
-      const long long avail = chunk_end - cursor;
+    while (mask != 0ull && !r.drained) {
+      const long long avail = r.end - r.cursor;
       if (avail <= 0) {
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(a.queue, (unsigned long long)a.chunk);
-        base = __shfl(base, 0);
-        if ((long long)base >= a.total) {
-          drained = true;
-          break;
-        }
-        cursor = (long long)base;
-        chunk_end = min((long long)base + a.chunk, a.total);
+        if (!next_range(a, r, lane)) break;
         continue;
       }
       const int rank = lanes_below(mask);
       const bool take = need && rank < avail;
-      if (take) alive = emit<(F & F_TORUS) != 0>(a, cursor + rank, p, acc);
-      cursor += min((long long)__popcll(mask), avail);
+      if (take) alive = emit<(F & F_TORUS) != 0>(a, r.cursor + rank, p, acc);
+      r.cursor += min((long long)__popcll(mask), avail);
       need = need && !take;
       mask = __ballot(need);
     }
-    if (!__any(alive) && drained) break;
+    if (!__any(alive) && r.drained) break;
     if (alive) {
       alive = step<false, F>(a, p, acc, nullptr, nullptr);
       if (!alive) photon_end(a, p);
@@ -1207,9 +1241,7 @@ __global__ void __launch_bounds__(adj_block_of<F>())
     adjoint_kernel(Args a0, AdjArgs b) {
   double *sg = lds_cells;
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
-  if (threadIdx.x == 0) s_bounded = 0u;
-  if (threadIdx.x < RF_N) s_rare[threadIdx.x] = 0.0f;
-  if (threadIdx.x < 32) s_hint[threadIdx.x] = -1;
+  clear_block_cells();
   stage_nodes(a0.g);
   const Args a = stage_tables<F>(a0);
   __syncthreads();
@@ -1217,39 +1249,30 @@ __global__ void __launch_bounds__(adj_block_of<F>())
   Acc acc{};
   bool alive = false;
   const int lane = threadIdx.x & 63;
-  long long cursor = 0, chunk_end = 0;
-  bool drained = false;
+  Range r = first_range(a);
   for (;;) {
     bool need = !alive;
     unsigned long long mask = __ballot(need);
-    while (mask != 0ull && !drained) {
-      const long long avail = chunk_end - cursor;
+    while (mask != 0ull && !r.drained) {
+      const long long avail = r.end - r.cursor;
       if (avail <= 0) {
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(a.queue, (unsigned long long)a.chunk);
-        base = __shfl(base, 0);
-        if ((long long)base >= a.total) {
-          drained = true;
-          break;
-        }
-        cursor = (long long)base;
-        chunk_end = min((long long)base + a.chunk, a.total);
+        if (!next_range(a, r, lane)) break;
         continue;
       }
       const int rank = lanes_below(mask);
       const bool take = need && rank < avail;
       if (take) {
-        p.gi = cursor + rank;
+        p.gi = r.cursor + rank;
         alive = emit<(F & F_TORUS) != 0>(a, p.gi, p, acc);
         p.pass = 0;
         p.T = p.Dsum = 0.0f;
         p.hasdep = false;
       }
-      cursor += min((long long)__popcll(mask), avail);
+      r.cursor += min((long long)__popcll(mask), avail);
       need = need && !take;
       mask = __ballot(need);
     }
-    if (!__any(alive) && drained) break;
+    if (!__any(alive) && r.drained) break;
     if (alive) {
       alive = step<true, F>(a, p, acc, &b, sg);
       if (!alive && p.pass == 0 && p.hasdep) {  // replay the photon from its counter, now adding the terms
@@ -1946,7 +1969,7 @@ static int fill_args(lh_model m, Args &a, const float *values, const float *ref,
   a.reach = m->g.reach;
   a.max_dist = c.max_distance > 0.0f ? c.max_distance : m->g.reach;
   a.max_vert = c.max_vertices > 0 ? c.max_vertices : (1 << 22);
-  a.chunk = c.chunk > 0 ? c.chunk : DEFAULT_CHUNK;
+  a.chunk = c.chunk;
   a.keep_zero = c.keep_zero_weight ? 1 : 0;
   a.reach_on = c.reach_bound ? 1 : 0;
   a.tally = tally;
@@ -2101,7 +2124,30 @@ static size_t place_lds(lh_model m, Args &a, const void *fn, int block, size_t c
   return end;
 }
 
-static void launch_adjoint(lh_model m, const Args &a, const AdjArgs &b, const lh_controls *ctl, size_t bytes,
+// How a launch's photons are handed out (Range).  An explicit chunk is every range's size.  Else, by the photons a
+// wavefront gets when all are handed out at once: up to STATIC_SHARE the first ranges hold them all, no queue, the
+// photons on as many wavefronts as there are (tank, 100,003 photons: 0.14 ms, 0.28 in chunks of 256 that fill an
+// eighth of the wavefronts; the tutorial's 2^18: 0.05 against 0.08); beyond it the first ranges hold three quarters
+// and the queue evens out the rest in small chunks (tank, 2^22 photons: 1.28 ms, 1.42 in chunks of 256 from the start,
+// whose last ones the launch waits for; 2^24: 4.69 against 4.77).  At the line both take the same (tank, 2^20: 0.44
+// and 0.43 ms).  Chunks of 64 to 128: below, the claims (12 ns each, one address) show on cheap photons.
+constexpr long long STATIC_SHARE = 384;
+constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
+
+static void claim_schedule(Args &a, const lh_controls *ctl, int grid, int block, hipStream_t st) {
+  const long long waves = (long long)grid * (block / 64);
+  long long first = a.chunk;
+  if (!(ctl && ctl->chunk > 0)) {
+    const long long share = (a.total + waves - 1) / waves;
+    first = share <= STATIC_SHARE ? share : share / 4 * 3;
+    a.chunk = (int)std::min(std::max(share / 16, MIN_CHUNK), MAX_CHUNK);
+  }
+  a.first_chunk = first;
+  a.dyn_at = std::min(a.total, waves * first);
+  if (a.dyn_at < a.total) hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue);
+}
+
+static void launch_adjoint(lh_model m, Args &a, const AdjArgs &b, const lh_controls *ctl, size_t bytes,
                            hipStream_t st) {
   const unsigned f = features_of(m, a, true) | (a.g.lds_nodes ? 0u : F_GNODES);
   const int grid = grid_of(m, ctl, kernel_of(true, f), bytes, block_for(true, f));
@@ -2109,6 +2155,7 @@ static void launch_adjoint(lh_model m, const Args &a, const AdjArgs &b, const lh
   m->last_launch[1] = grid / std::max(m->cus, 1);
   m->last_launch[2] = (int32_t)bytes;
   m->last_launch[7] = (int32_t)f | 0x100;
+  claim_schedule(a, ctl, grid, block_for(true, f), st);
   launch_kernel(true, f, dim3(grid), bytes, st, a, b, 0);
 }
 
@@ -2121,13 +2168,13 @@ static void launch_trace(lh_model m, Args &a, int n_events, const lh_controls *c
       place_lds(m, a, fn, block_for(false, f), cells <= LDS_TALLY_CELLS ? (size_t)cells * sizeof(double) : 0,
                 true, ctl);
   const int n_lds = a.lds_tally ? (int)cells : 0;
-  hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue);
   const unsigned fk = f | (a.g.lds_nodes ? 0u : F_GNODES);  // the walk reads its nodes from LDS or from memory
   const int grid = grid_of(m, ctl, kernel_of(false, fk), bytes, block_for(false, fk));
   m->last_launch[0] = grid;
   m->last_launch[1] = grid / std::max(m->cus, 1);
   m->last_launch[2] = (int32_t)bytes;
   m->last_launch[7] = (int32_t)fk;
+  claim_schedule(a, ctl, grid, block_for(false, fk), st);
   launch_kernel(false, fk, dim3(grid), bytes, st, a, AdjArgs{}, n_lds);
 }
 
@@ -2248,8 +2295,6 @@ LH_API int lh_adjoint(lh_model m, const float *values, const float *ref, int64_t
   a.nsrc = n_sources;
   a.total = total;
   AdjArgs b{cot, slots, grad, n_grad};
-  hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, m->queue);
-  HIP_TRY(hipGetLastError());
   const int slot = (int)(m->launches % TIME_RING);
   HIP_TRY(hipEventRecord(m->ev0[slot], st));
   const size_t bytes = place_lds(m, a, kernel_of(true, features_of(m, a, true)), block_for(true, features_of(m, a, true)),
@@ -2360,7 +2405,6 @@ LH_API int lh_batch_adjoint(lh_batch b, const float *values, const float *ref, i
   a.total = b->total;
   a.queue = b->queue;
   AdjArgs g{cot, b->slots, grad, n_grad};
-  hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue);
   const size_t bytes = place_lds(m, a, kernel_of(true, features_of(m, a, true)), block_for(true, features_of(m, a, true)),
                                  (size_t)n_grad * sizeof(double), false, ctl);
   launch_adjoint(m, a, g, ctl, bytes, st);
