@@ -206,6 +206,25 @@ int lh_adjoint(lh_model model, const float *values_dev, const float *ref_values_
                const lh_controls *controls, const double *cotangent_dev, int32_t n_events, double *grad_dev,
                int32_t n_grad, double *health_dev, void *stream);
 
+/* The same derivative from a tape of each photon's path.  lh_trace_tape is lh_trace at the values themselves, and writes
+ * the tape where *by_adjoint is 0; lh_adjoint_tape is lh_adjoint with the paths read from it, after writing it with one
+ * walk of its own where *by_adjoint is 1 (a surface row can draw a facet path; `tape_dev` is then scratch of this call,
+ * and the trace is lh_trace).  lh_tape_size gives the bytes for a launch of `photons` photons, 0 where it takes no tape
+ * (reference values, more than 2^26 photons, a time grid, Mie lobes, CE knots, torus leaves, deposits at the emission,
+ * `jump`, `reach_bound`): use lh_trace and lh_adjoint there.  The tape is the caller's, 16-byte aligned, and holds one
+ * launch: values, sources, seed and controls of the adjoint are the trace's.  Photons that it has no room for are
+ * replayed.  `health_dev` of the adjoint counts every photon once; its other cells are those of the replays.  No
+ * counterpart in the reference. */
+int lh_tape_size(lh_model model, const lh_controls *controls, int32_t has_ref, int64_t photons, int64_t *bytes,
+                 int32_t *by_adjoint);
+int lh_trace_tape(lh_model model, const float *values_dev, int64_t n_values, const lh_source *sources,
+                  int32_t n_sources, uint64_t seed, const lh_controls *controls, double *tally_dev, int32_t n_events,
+                  double *health_dev, void *tape_dev, int64_t tape_bytes, void *stream);
+int lh_adjoint_tape(lh_model model, const float *values_dev, int64_t n_values, const int32_t *slots_dev,
+                    const lh_source *sources, int32_t n_sources, uint64_t seed, const lh_controls *controls,
+                    const double *cotangent_dev, int32_t n_events, double *grad_dev, int32_t n_grad,
+                    double *health_dev, void *tape_dev, int64_t tape_bytes, void *stream);
+
 /* A staged batch, for launches a caller captures in a HIP graph.  lh_batch_create uploads and checks the sources
  * (and, for the adjoint, the gradient slots: NULL slots_dev for a forward-only batch); it allocates and may
  * synchronise.  lh_batch_trace / lh_batch_adjoint then only enqueue kernels on `stream` (no allocation, no host
@@ -224,6 +243,14 @@ int lh_batch_trace(lh_batch batch, const float *values_dev, const float *ref_val
 int lh_batch_adjoint(lh_batch batch, const float *values_dev, const float *ref_values_dev, int64_t n_values,
                      uint64_t seed, const lh_controls *controls, const double *cotangent_dev, int32_t n_events,
                      double *grad_dev, int32_t n_grad, double *health_dev, void *stream);
+
+/* ... with a tape: lh_tape_size of the batch's photons. */
+int lh_batch_trace_tape(lh_batch batch, const float *values_dev, int64_t n_values, uint64_t seed,
+                        const lh_controls *controls, double *tally_dev, int32_t n_events, double *health_dev,
+                        void *tape_dev, int64_t tape_bytes, void *stream);
+int lh_batch_adjoint_tape(lh_batch batch, const float *values_dev, int64_t n_values, uint64_t seed,
+                          const lh_controls *controls, const double *cotangent_dev, int32_t n_events, double *grad_dev,
+                          int32_t n_grad, double *health_dev, void *tape_dev, int64_t tape_bytes, void *stream);
 
 /* The navigator on n rays (device arrays): from x (n*3) along d (n*3) in navigator id vol (-1: located here), the
  * photon sitting on face `last` (-1: none), the next visible crossing within tmax (<= 0: the reach): its distance

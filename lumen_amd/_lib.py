@@ -62,6 +62,7 @@ _LIB = None
 SYMBOLS = ("lh_model_create", "lh_model_destroy", "lh_model_info", "lh_trace", "lh_adjoint", "lh_query",
            "lh_batch_create", "lh_batch_destroy", "lh_batch_trace", "lh_batch_adjoint", "lh_last_kernel_ms",
            "lh_last_launch", "lh_model_jump", "lh_bvh_build", "lh_launches", "lh_kernel_ms_of", "lh_trace_static",
+           "lh_tape_size", "lh_trace_tape", "lh_adjoint_tape", "lh_batch_trace_tape", "lh_batch_adjoint_tape",
            "lh_last_error")
 
 
@@ -94,6 +95,16 @@ def lib():
         L.lh_batch_adjoint.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_uint64,
                                        C.POINTER(LhControls), C.c_void_p, C.c_int32, C.c_void_p, C.c_int32,
                                        C.c_void_p, C.c_void_p]
+        ctl, tape = C.POINTER(LhControls), [C.c_void_p, C.c_int64, C.c_void_p]
+        L.lh_tape_size.argtypes = [C.c_void_p, ctl, C.c_int32, C.c_int64, C.POINTER(C.c_int64), _i]
+        L.lh_trace_tape.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.POINTER(LhSource), C.c_int32, C.c_uint64, ctl,
+                                    C.c_void_p, C.c_int32, C.c_void_p] + tape
+        L.lh_adjoint_tape.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.POINTER(LhSource), C.c_int32,
+                                      C.c_uint64, ctl, C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p] + tape
+        L.lh_batch_trace_tape.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_uint64, ctl, C.c_void_p, C.c_int32,
+                                          C.c_void_p] + tape
+        L.lh_batch_adjoint_tape.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_uint64, ctl, C.c_void_p, C.c_int32,
+                                            C.c_void_p, C.c_int32, C.c_void_p] + tape
         L.lh_last_kernel_ms.argtypes = [C.c_void_p, _f]
         L.lh_launches.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
         L.lh_kernel_ms_of.argtypes = [C.c_void_p, C.c_int64, _f]

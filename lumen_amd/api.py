@@ -318,6 +318,22 @@ class Engine:
         _lib.check(_lib.lib().lh_launches(self.handle, _lib.C.byref(n)), "lh_launches")
         return n.value
 
+    def tape(self, ctl, has_ref: bool, photons: int, adjoint: bool):
+        """Return a tape (a uint8 device tensor) for a launch of ``photons`` photons whose adjoint follows
+        (``adjoint``: for its adjoint), or None where that launch writes none or the device has no room for it (the
+        adjoint then replays the photons)."""  # noqa: D205, D209
+        import torch
+
+        size, by_adjoint = _lib.C.c_int64(), _lib.C.c_int32()
+        _lib.check(_lib.lib().lh_tape_size(self.handle, _lib.C.byref(ctl), int(has_ref), int(photons),
+                                           _lib.C.byref(size), _lib.C.byref(by_adjoint)), "lh_tape_size")
+        if size.value == 0 or bool(by_adjoint.value) != adjoint:
+            return None
+        try:
+            return torch.empty(size.value, dtype=torch.uint8, device=self.device)
+        except torch.cuda.OutOfMemoryError:
+            return None
+
     def upload(self, values: np.ndarray):
         """Return the packed values on the device, the previous upload again when they are the same (a copy from
         pageable memory waits for the stream; unchanged values need none)."""  # noqa: D205, D209

@@ -3,11 +3,12 @@
     params_t = {"materials/Water/ABSLENGTH": torch.tensor(..., requires_grad=True), ...}
     light = simulate_diff(det, source, params_t, samples=2**24, seed=0)
     loss = f(light.arrivals, light.charge)            # any torch function of the tallies
-    loss.backward()                                   # lh_adjoint: one replayed walk pair per photon
+    loss.backward()                                   # lh_adjoint_tape: from the photons' paths
 
 The keys' values are scattered into the packed values (``lumen_amd.pack``) by differentiable torch indexing; the
-photon loop's forward is ``lh_trace`` and its backward ``lh_adjoint`` (the photons replayed from their Philox
-counters, no stored paths).  Every random choice is drawn at the reference values (default: the values given,
+photon loop's backward reads the photons' paths from a tape that the forward wrote (``lh_trace_tape``), or where a
+surface can draw facets from one it writes itself (``lh_adjoint_tape``); a launch that takes no tape is replayed from
+its Philox counters (``lh_adjoint``).  Every random choice is drawn at the reference values (default: the values given,
 detached), as the reference's derivative is (``api.py:748-787``, ``transport/estimator.py``): the gradient is the
 derivative of the light at a fixed seed, which common-random-number finite differences converge to.  Sensor values
 (QE, efficiency) act after tracking: their derivatives are ordinary torch autograd on the readout.
@@ -49,7 +50,7 @@ _Run.kernel_ms = _lazy("kernel_ms", float)
 _Run.adjoint_ms = _lazy("adjoint_ms", float)
 
 
-def _trace(run: _Run, values):
+def _trace(run: _Run, values, tape=None):
     import torch
 
     eng = run.eng
@@ -58,19 +59,24 @@ def _trace(run: _Run, values):
     st = torch.cuda.current_stream(eng.device)
     ctl = run.controls.struct()
     ref = run.ref_values
-    _lib.check(_lib.lib().lh_trace(eng.handle, _lib.C.c_void_p(values.data_ptr()),
-                                   None if ref is None else _lib.C.c_void_p(ref.data_ptr()), int(values.numel()),
-                                   run.rows, len(run.rows), _lib.C.c_uint64(run.seed), _lib.C.byref(ctl),
-                                   _lib.C.c_void_p(tally.data_ptr()), run.n_ev, _lib.C.c_void_p(health.data_ptr()),
-                                   _lib.C.c_void_p(st.cuda_stream)), "lh_trace")
+    vp = _lib.C.c_void_p
+    rest = (int(values.numel()), run.rows, len(run.rows), _lib.C.c_uint64(run.seed), _lib.C.byref(ctl),
+            vp(tally.data_ptr()), run.n_ev, vp(health.data_ptr()))
+    if tape is None:
+        _lib.check(_lib.lib().lh_trace(eng.handle, vp(values.data_ptr()), None if ref is None else vp(ref.data_ptr()),
+                                       *rest, vp(st.cuda_stream)), "lh_trace")
+    else:
+        _lib.check(_lib.lib().lh_trace_tape(eng.handle, vp(values.data_ptr()), *rest, vp(tape.data_ptr()),
+                                            int(tape.numel()), vp(st.cuda_stream)), "lh_trace_tape")
     run.health = health
     launch = eng.launches() - 1
     run.kernel_ms = lambda: eng.kernel_ms(launch)
     return tally
 
 
-def adjoint(run: _Run, values, cot):
-    """Return the gradient slots (n_grad,) float64 of the loss whose cotangent on the tallies is ``cot``."""
+def adjoint(run: _Run, values, cot, tape=None):
+    """Return the gradient slots (n_grad,) float64 of the loss whose cotangent on the tallies is ``cot``; ``tape``:
+    of these photons' paths (None: they are replayed)."""  # noqa: D205, D209
     import torch
 
     eng = run.eng
@@ -80,36 +86,50 @@ def adjoint(run: _Run, values, cot):
     st = torch.cuda.current_stream(eng.device)
     ctl = run.controls.struct()
     ref = run.ref_values
-    _lib.check(_lib.lib().lh_adjoint(eng.handle, _lib.C.c_void_p(values.data_ptr()),
-                                     None if ref is None else _lib.C.c_void_p(ref.data_ptr()), int(values.numel()),
-                                     _lib.C.c_void_p(run.slots.data_ptr()), run.rows, len(run.rows),
-                                     _lib.C.c_uint64(run.seed), _lib.C.byref(ctl), _lib.C.c_void_p(cot.data_ptr()),
-                                     run.n_ev, _lib.C.c_void_p(grad.data_ptr()), max(run.n_grad, 1),
-                                     _lib.C.c_void_p(health.data_ptr()), _lib.C.c_void_p(st.cuda_stream)),
-               "lh_adjoint")
+    vp = _lib.C.c_void_p
+    rest = (int(values.numel()), vp(run.slots.data_ptr()), run.rows, len(run.rows), _lib.C.c_uint64(run.seed),
+            _lib.C.byref(ctl), vp(cot.data_ptr()), run.n_ev, vp(grad.data_ptr()), max(run.n_grad, 1),
+            vp(health.data_ptr()))
+    if tape is None:
+        _lib.check(_lib.lib().lh_adjoint(eng.handle, vp(values.data_ptr()),
+                                         None if ref is None else vp(ref.data_ptr()), *rest, vp(st.cuda_stream)),
+                   "lh_adjoint")
+    else:
+        _lib.check(_lib.lib().lh_adjoint_tape(eng.handle, vp(values.data_ptr()), *rest, vp(tape.data_ptr()),
+                                              int(tape.numel()), vp(st.cuda_stream)), "lh_adjoint_tape")
     run.adj_health = health
     launch = eng.launches() - 1
     run.adjoint_ms = lambda: eng.kernel_ms(launch)
     return grad[: run.n_grad]
 
 
+def _tape(run: _Run, by_adjoint: bool):
+    return run.eng.tape(run.controls.struct(), run.ref_values is not None, sum(r.n for r in run.rows), by_adjoint)
+
+
 def _function():
     import torch
 
     class PhotonLoop(torch.autograd.Function):
-        """tally = photon_loop(values): forward lh_trace, backward lh_adjoint."""
+        """tally = photon_loop(values): forward lh_trace, backward lh_adjoint.  Where the launch takes a tape, the
+        forward of a detector without facet paths writes it (saved beside the values), else the backward itself."""
 
         @staticmethod
         def forward(ctx, values, run):
             ctx.run = run
-            ctx.save_for_backward(values)
-            return _trace(run, values.detach().contiguous())
+            tape = None
+            if ctx.needs_input_grad[0]:
+                tape = _tape(run, False)
+            ctx.save_for_backward(values, tape)
+            return _trace(run, values.detach().contiguous(), tape)
 
         @staticmethod
         def backward(ctx, g):
-            (values,) = ctx.saved_tensors
+            values, tape = ctx.saved_tensors
             run = ctx.run
-            gs = adjoint(run, values.detach().contiguous(), g)
+            if tape is None:
+                tape = _tape(run, True)
+            gs = adjoint(run, values.detach().contiguous(), g, tape)
             gv = torch.zeros(values.shape, dtype=torch.float64, device=values.device)
             gv[run.first_index] = gs[run.first_slot]  # the copies of a slot share one value of the key
             return gv.to(values.dtype), None
@@ -179,7 +199,7 @@ def simulate_diff(det, source, params_t: dict, *, samples=None, seed=0, params: 
                      samples if not hasattr(source, "sources") else None, source)
     light.kernel_ms = lambda: run.kernel_ms
     light.group_specs = list(det.groups or [])
-    light.provenance = dict(seed=int(seed), samples=samples, detector=det.name, derivative="adjoint (replay)",
+    light.provenance = dict(seed=int(seed), samples=samples, detector=det.name, derivative="adjoint",
                             keys=keys, run=run)
     return light
 

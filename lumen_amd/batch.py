@@ -61,11 +61,12 @@ class BatchRun:
             self.eng.ensure_jump()
         self._g_fwd = self._g_both = None
         self._loss = None
+        self._tape = None  # forward_adjoint's: the photons' paths, for its adjoint
 
     def close(self):
         """Release the batch's device buffers (its sources and work queue); the captured graphs go with them."""
         if getattr(self, "handle", None):
-            self._g_fwd = self._g_both = None
+            self._g_fwd = self._g_both = self._tape = None
             _lib.lib().lh_batch_destroy(self.handle)
             self.handle = None
 
@@ -76,40 +77,49 @@ class BatchRun:
             pass
 
     # ------------------------------------------------------------------------------------------ raw launches
-    def _launch(self, ctl=None):
+    def _launch(self, ctl=None, tape=None):
         import torch
 
         st = torch.cuda.current_stream(self.eng.device)
         c = (ctl or self.controls).struct()
-        _lib.check(_lib.lib().lh_batch_trace(self.handle, _lib.C.c_void_p(self.values.data_ptr()), None,
-                                             int(self.values.numel()), _lib.C.c_uint64(self.seed), _lib.C.byref(c),
-                                             _lib.C.c_void_p(self.tally.data_ptr()), self.n_ev,
-                                             _lib.C.c_void_p(self.health.data_ptr()), _lib.C.c_void_p(st.cuda_stream)),
-                   "lh_batch_trace")
+        vp = _lib.C.c_void_p
+        rest = (int(self.values.numel()), _lib.C.c_uint64(self.seed), _lib.C.byref(c), vp(self.tally.data_ptr()),
+                self.n_ev, vp(self.health.data_ptr()))
+        if tape is None:
+            _lib.check(_lib.lib().lh_batch_trace(self.handle, vp(self.values.data_ptr()), None, *rest,
+                                                 vp(st.cuda_stream)), "lh_batch_trace")
+        else:
+            _lib.check(_lib.lib().lh_batch_trace_tape(self.handle, vp(self.values.data_ptr()), *rest,
+                                                      vp(tape.data_ptr()), int(tape.numel()), vp(st.cuda_stream)),
+                       "lh_batch_trace_tape")
 
-    def _launch_adjoint(self, ctl=None):
+    def _launch_adjoint(self, ctl=None, tape=None):
         import torch
 
         st = torch.cuda.current_stream(self.eng.device)
         c = (ctl or self.adj_controls or Controls()).struct()
-        _lib.check(_lib.lib().lh_batch_adjoint(self.handle, _lib.C.c_void_p(self.values.data_ptr()), None,
-                                               int(self.values.numel()), _lib.C.c_uint64(self.seed), _lib.C.byref(c),
-                                               _lib.C.c_void_p(self.cot.data_ptr()), self.n_ev,
-                                               _lib.C.c_void_p(self.grad.data_ptr()), self.n_grad,
-                                               _lib.C.c_void_p(self.adj_health.data_ptr()),
-                                               _lib.C.c_void_p(st.cuda_stream)), "lh_batch_adjoint")
+        vp = _lib.C.c_void_p
+        rest = (int(self.values.numel()), _lib.C.c_uint64(self.seed), _lib.C.byref(c), vp(self.cot.data_ptr()),
+                self.n_ev, vp(self.grad.data_ptr()), self.n_grad, vp(self.adj_health.data_ptr()))
+        if tape is None:
+            _lib.check(_lib.lib().lh_batch_adjoint(self.handle, vp(self.values.data_ptr()), None, *rest,
+                                                   vp(st.cuda_stream)), "lh_batch_adjoint")
+        else:
+            _lib.check(_lib.lib().lh_batch_adjoint_tape(self.handle, vp(self.values.data_ptr()), *rest,
+                                                        vp(tape.data_ptr()), int(tape.numel()), vp(st.cuda_stream)),
+                       "lh_batch_adjoint_tape")
 
-    def _fwd_body(self, ctl=None):
+    def _fwd_body(self, ctl=None, tape=None):
         self.tally.zero_()  # a fill kernel (graph-safe), not a memset
         self.health.zero_()
-        self._launch(ctl)
+        self._launch(ctl, tape)
 
     def _both_body(self):
-        self._fwd_body()
+        self._fwd_body(tape=self._tape)
         self.cot.copy_(self._loss(self.tally))
         self.grad.zero_()
         self.adj_health.zero_()
-        self._launch_adjoint()
+        self._launch_adjoint(tape=self._tape)
 
     def _capture(self, body):
         import torch
@@ -141,6 +151,13 @@ class BatchRun:
         slots (n_grad,).  Captured as one graph on first use (the loss function is part of it)."""  # noqa: D205, D209
         if self._loss is not loss:
             self._loss, self._g_both = loss, None
+        if self._tape is None and self._g_both is None and self.has_grad:
+            ctl = self.controls.struct()
+            self._tape = self.eng.tape(ctl, False, self.total, False)
+            if self._tape is None:
+                self._tape = self.eng.tape(ctl, False, self.total, True)
+        if self.adj_controls is None and self._tape is not None:
+            self.adj_controls = Controls()  # the adjoint reads the tape: no walk whose launch shape matters
         if self.adj_controls is None:  # the adjoint's launch shape: tuned once, with this loss's cotangent
             self._fwd_body()
             self.cot.copy_(loss(self.tally))

@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "liblumen_hip.so")
 SOURCES = [os.path.join(HERE, "csrc", f) for f in ("engine.hip", "unified_tables.cpp", "bvh_build.cpp")]
-DEPS = SOURCES + [os.path.join(HERE, "csrc", f) for f in ("nav.h", "optics.h", "philox.h", "adjoint.h", "unified.h")] + [
+DEPS = SOURCES + [os.path.join(HERE, "csrc", f) for f in ("nav.h", "optics.h", "philox.h", "adjoint.h", "tape.h", "unified.h")] + [
     os.path.join(ROOT, "include", "lumen_hip.h")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("LUMEN_ARCH", "gfx950")

@@ -28,6 +28,7 @@
 #include "nav.h"
 #include "optics.h"
 #include "philox.h"
+#include "tape.h"
 #include "unified.h"
 
 namespace lh_host {
@@ -63,6 +64,9 @@ constexpr int OCC_CACHE = 8;
 // a kernel's features (template parameter): separate reference values, bulk channels beyond Rayleigh (Mie,
 // WLS), the time histogram, BVH nodes read from global memory
 constexpr unsigned F_REF = 1, F_CHAN = 2, F_TIME = 4, F_GNODES = 8, F_TORUS = 16, F_REACH = 32;
+// ... and a tape written for the adjoint (tape.h), of a plain run or of one with a WLS channel: by the forward, or
+// (F_PATH) by a walk of the adjoint's own that adds no tallies and takes the facet paths' derivatives
+constexpr unsigned F_TAPE = 64, F_PATH = 128;
 // the features an adjoint kernel is specialised on
 constexpr unsigned F_ADJ_MASK = F_REF | F_CHAN | F_GNODES | F_TORUS | F_REACH;
 
@@ -114,6 +118,9 @@ struct Args {
   // detected share to the sensor of the volume left (an exit sensor), and per class the row whose detected share a
   // photon emitted inside a sensor volume of that class deposits at its emission (-1: none)
   int left_at, born_at;
+  Tape tape;             // the forward's tape (F_TAPE)
+  const unsigned *replay;  // the adjoint's: the launch indices a tape left to the replay, their number before them
+                           // (null: every photon)
 };
 
 struct Photon {
@@ -137,6 +144,8 @@ struct Photon {
   float T, Dsum;
   bool hasdep;
   RateD da, dr, dm, dw;
+  TapePos tape;  // the forward's place on the tape and its step's record (F_TAPE)
+  TapeRec rec;
 };
 
 struct Acc {  // per-lane health accumulators of the frequent fates, flushed once per launch
@@ -394,6 +403,13 @@ __device__ inline bool emit(const Args &a, long long gi, Photon &p, Acc &acc) {
   return true;
 }
 
+// x as a value of its own: the compiler neither merges nor contracts across it
+__device__ __forceinline__ float apart(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ float3 apart(float3 v) { return mk3(apart(v.x), apart(v.y), apart(v.z)); }
+
 // Geant4's unified facet path (facets.py:318-397): facets drawn for the current direction and mirrored about
 // until the direction leaves the surface; the polarisation mirrored about each facet's half vector.  The path is
 // drawn at the reference width `sigma`; with `ratio` its log density ratio live / reference is added to logw
@@ -586,9 +602,10 @@ __device__ inline void medium_cache(const Args &a, Photon &p, const AdjArgs *b) 
 }
 
 // the cotangent of one deposit at sensor s: dLoss/d(arrival) plus the charge cells' at its wavelength and angle
-__device__ inline float deposit_cotangent(const Args &a, const AdjArgs *b, const Photon &p, int s, float theta) {
-  const double *c = b->cot + (long long)p.event * a.tally_stride;
-  const Cells cl = charge_cells(a, p.lam, theta);
+__device__ inline float deposit_cotangent(const Args &a, const AdjArgs *b, int event, float lam, int s,
+                                          float theta) {
+  const double *c = b->cot + (long long)event * a.tally_stride;
+  const Cells cl = charge_cells(a, lam, theta);
   const long long cb = 3LL * a.S + (long long)s * a.K + cl.base;
   double cw = c[s] + (double)((1.0f - cl.fl) * (1.0f - cl.ft)) * c[cb];
   if (cl.fl > 0.0f) cw += (double)(cl.fl * (1.0f - cl.ft)) * c[cb + a.Kt];
@@ -679,7 +696,7 @@ __device__ __forceinline__ void rates_add(double *sg, const Photon &p, float ka,
 // into the block's accumulators sg)
 template <bool ADJ, unsigned F>
 __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b, double *sg) {
-  constexpr bool REF = F & F_REF, CHAN = F & F_CHAN;
+  constexpr bool REF = F & F_REF, CHAN = F & F_CHAN, TAPE = !ADJ && (F & F_TAPE), PATH = F & F_PATH;
   const Geo &g = a.g;
   float b0 = band_at(maxabs3(p.x));
   if (p.nz >= ZERO_STEPS_BEFORE_PUSH) {  // G4Navigator's stuck-track push (step.py:269-282 `_recover`)
@@ -706,7 +723,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
         deposit<F>(a, p, acc, sensor, dep_q, p.t, theta);
         acc.surf += p.w * p.w0;
       } else {
-        const float D = dep_q * p.w0 * deposit_cotangent(a, b, p, sensor, theta);
+        const float D = dep_q * p.w0 * deposit_cotangent(a, b, p.event, p.lam, sensor, theta);
         if (D != 0.0f) {
           p.hasdep = true;
           if (p.pass == 1) {
@@ -752,6 +769,11 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
   const float reach_live = __expf(-mu * dist), reach_ref = REF ? __expf(-mu_r * dist) : reach_live;
   const float att = __expf(-ml.mu_abs * dist), att_r = REF ? __expf(-mr.mu_abs * dist) : att;
   const float v_g = C_VACUUM / ml.ng;
+  if (TAPE) {  // the step's record (tape.h), so far a deposit's
+    p.rec.len = apart(dist);
+    p.rec.free = p.rec.dep = p.rec.aux = 0.0f;
+    p.rec.code = tape_code(TAPE_DEPOSIT, 0, cont, cb * a.L[L_CLASSES] + (ca < 0 ? 0 : ca), 0);
+  }
   SurfEval sl, sr;
   int o = -1;
   float pprop[N_OUT], pdraw[N_OUT];
@@ -802,9 +824,13 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
     if (sensor >= 0 && !cont) {
       const float theta = a.Kt > 1 ? cathode_theta(g, vs, fma3(dist, p.d, p.x)) : 0.0f;
       if (!ADJ) {
-        deposit<F>(a, p, acc, sensor, dep_q, p.t + dist / v_g, theta);
+        if (!PATH) deposit<F>(a, p, acc, sensor, dep_q, p.t + dist / v_g, theta);
+        if (TAPE) {
+          p.rec.dep = apart(dep_q) * apart(p.w0);
+          p.rec.code |= (unsigned)sensor << 18;
+        }
       } else {
-        const float D = dep_q * p.w0 * deposit_cotangent(a, b, p, sensor, theta);
+        const float D = dep_q * p.w0 * deposit_cotangent(a, b, p.event, p.lam, sensor, theta);
         if (D != 0.0f) {
           p.hasdep = true;
           if (p.pass == 1) {  // the deposit's own factors: reach, attenuation, the detected share
@@ -843,6 +869,11 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
       const float kc = mc > 0.0f ? 1.0f / mc : 0.0f;
       rates_add<CHAN>(sg, p, -s, (ch == 0 ? kc : 0.0f) - s, (ch == 1 ? kc : 0.0f) - s, (ch == 2 ? kc : 0.0f) - s,
                       ahead);
+    }
+    if (TAPE) {
+      p.rec.free = apart(s);
+      p.rec.aux = apart(mc);
+      p.rec.code = tape_event(p.rec.code, TAPE_SCATTER, ch);
     }
     p.x = fma3(s, p.d, p.x);
     p.t += s / v_g;
@@ -935,6 +966,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
       }
     }
     if (ok) {
+      if (TAPE) p.rec.code = tape_event(p.rec.code, TAPE_SURFACE, o);
       const float w_if = w_at * att * ratio(pick6(sl.p, o), pick6(pprop, o));
       const float r_o = ratio(pick6(pdraw, o), pick6(pprop, o));
       wr_new = p.wr * (reach_ref != 0.0f ? 1.0f : 0.0f) * att_r * r_o;
@@ -965,17 +997,19 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
           const bool cover = sr.flags & FLAG_COVER, weigh = want_ratio || cover;
           if (sr.flags & FLAG_REFRACTS) {
             const float n2l = index_at(a.L, a.P, class_medium(a, ca), p.lam);
-            dn = glisur_dielectric(rng, p.vertex, sr.sigma, sl.sigma, cover, weigh, adj_event, wi, n, ml.n, n2l,
+            dn = glisur_dielectric(rng, p.vertex, sr.sigma, sl.sigma, cover, weigh, PATH || adj_event, wi, n, ml.n, n2l,
                                    er0, ei0, logw, dlogw, far);
           } else {
-            dn = glisur_metal(rng, p.vertex, sr.sigma, sl.sigma, cover, weigh, adj_event, wi, n, er0, ei0, logw,
+            dn = glisur_metal(rng, p.vertex, sr.sigma, sl.sigma, cover, weigh, PATH || adj_event, wi, n, er0, ei0, logw,
                               dlogw);
           }
           if (weigh) w_lobe = __expf(logw);
         } else {
-          dn = facet_path(p, rng, sr.sigma, sl.sigma, a.ut, want_ratio, adj_event, wi, n, er0, ei0, logw, dlogw);
+          dn = facet_path(p, rng, sr.sigma, sl.sigma, a.ut, want_ratio, PATH || adj_event, wi, n, er0, ei0, logw,
+                          dlogw);
           if (want_ratio) w_lobe = __expf(logw);
         }
+        if (PATH) p.rec.aux = dlogw;
         if (adj_event) {  // the live log density's derivative in the width: sigma_alpha, or -d/dr for polish
           const int col = glisur ? COL_POLISH : COL_SIGMA;
           const float sgn = glisur ? -1.0f : 1.0f;
@@ -1086,7 +1120,11 @@ __device__ __forceinline__ void clear_block_cells() {
   if (threadIdx.x < 32) s_hint[threadIdx.x] = -1;
 }
 
-__global__ void reset_queue(unsigned long long *q) { *q = 0ull; }
+// the work queue at a launch's start, and a tape's count of pool chunks (the forward) or of its replay's list
+__global__ void reset_queue(unsigned long long *q, unsigned *count) {
+  *q = 0ull;
+  if (count) *count = 0u;
+}
 
 // the navigator on given rays: the next visible crossing (t, the navigator id entered, the normal) and the volume
 // holding each ray's start
@@ -1167,9 +1205,17 @@ __device__ __forceinline__ Range first_range(const Args &a) {
   return Range{b, min(b + a.first_chunk, a.dyn_at), false};
 }
 
+// ... and of the photons a tape left to the replay: as many of the list for every wavefront
+__device__ __forceinline__ Range replay_range(const Args &a) {
+  const unsigned waves = gridDim.x * (blockDim.x >> 6), n = a.replay[0], share = (n + waves - 1) / waves;
+  const unsigned w = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+  const unsigned b = min(w * share, n);
+  return Range{(long long)b, (long long)min(b + share, n), false};
+}
+
 // the next chunk when the range is used up: false once there is none
 __device__ __forceinline__ bool next_range(const Args &a, Range &r, int lane) {
-  if (a.dyn_at < a.total) {
+  if (a.dyn_at < a.total && !a.replay) {
     unsigned long long c = 0;
     if (lane == 0) c = atomicAdd(a.queue, (unsigned long long)a.chunk);
     const long long base = a.dyn_at + (long long)__shfl(c, 0);
@@ -1188,6 +1234,9 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
   if (a0.lds_tally)
     for (int i = threadIdx.x; i < n_lds; i += blockDim.x) lds_cells[i] = 0.0;
   clear_block_cells();
+  if constexpr ((F & F_TAPE) != 0) {
+    if (threadIdx.x < 16) s_pool[threadIdx.x][0] = s_pool[threadIdx.x][1] = 0u;
+  }
   stage_nodes(a0.g);
   const Args a = stage_tables<F>(a0);
   __syncthreads();
@@ -1208,7 +1257,14 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
       }
       const int rank = lanes_below(mask);
       const bool take = need && rank < avail;
-      if (take) alive = emit<(F & F_TORUS) != 0>(a, r.cursor + rank, p, acc);
+      if (take) {
+        alive = emit<(F & F_TORUS) != 0>(a, r.cursor + rank, p, acc);
+        if constexpr ((F & F_TAPE) != 0) {
+          p.gi = r.cursor + rank;
+          tape_begin(p.tape, (unsigned)p.gi, p.lam);
+          if (!alive) tape_end(a.tape, p.tape, (unsigned)p.gi, p.event);
+        }
+      }
       r.cursor += min((long long)__popcll(mask), avail);
       need = need && !take;
       mask = __ballot(need);
@@ -1216,10 +1272,14 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
     if (!__any(alive) && r.drained) break;
     if (alive) {
       alive = step<false, F>(a, p, acc, nullptr, nullptr);
-      if (!alive) photon_end(a, p);
+      if constexpr ((F & F_TAPE) != 0) tape_step<(F & F_CHAN) != 0, (F & F_PATH) != 0>(a.tape, p.tape, p.rec, p.lam);
+      if (!alive) {
+        if constexpr ((F & F_PATH) == 0) photon_end(a, p);
+        if constexpr ((F & F_TAPE) != 0) tape_end(a.tape, p.tape, (unsigned)p.gi, p.event);
+      }
     }
   }
-  flush_health(a, acc);
+  if constexpr ((F & F_PATH) == 0) flush_health(a, acc);
   if (a.lds_tally) {  // one global atomic per touched cell per block
     __syncthreads();
     for (int i = threadIdx.x; i < n_lds; i += blockDim.x)
@@ -1239,6 +1299,7 @@ template <unsigned F>
 __global__ void __launch_bounds__(adj_block_of<F>())
     __attribute__((amdgpu_waves_per_eu(LH_ADJ_WAVES_PER_EU)))
     adjoint_kernel(Args a0, AdjArgs b) {
+  if (a0.replay && a0.replay[0] == 0u) return;
   double *sg = lds_cells;
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
   clear_block_cells();
@@ -1249,7 +1310,7 @@ __global__ void __launch_bounds__(adj_block_of<F>())
   Acc acc{};
   bool alive = false;
   const int lane = threadIdx.x & 63;
-  Range r = first_range(a);
+  Range r = a.replay ? replay_range(a) : first_range(a);
   for (;;) {
     bool need = !alive;
     unsigned long long mask = __ballot(need);
@@ -1262,7 +1323,7 @@ __global__ void __launch_bounds__(adj_block_of<F>())
       const int rank = lanes_below(mask);
       const bool take = need && rank < avail;
       if (take) {
-        p.gi = r.cursor + rank;
+        p.gi = a.replay ? (long long)a.replay[1 + r.cursor + rank] : r.cursor + rank;
         alive = emit<(F & F_TORUS) != 0>(a, p.gi, p, acc);
         p.pass = 0;
         p.T = p.Dsum = 0.0f;
@@ -1289,6 +1350,170 @@ __global__ void __launch_bounds__(adj_block_of<F>())
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x)
     if (sg[i] != 0.0) unsafeAtomicAdd(b.grad + i, sg[i]);
   flush_health(a, acc);
+}
+
+// the adjoint from a tape (tape.h): every photon's records read twice, in the walk's order, the same terms as the
+// replay adds from the same operands.  A lane takes the next photon of its wavefront's range that has a deposit.
+constexpr int TAPE_BLOCK = 256;
+
+// a photon's records in order
+struct TapeReader {
+  unsigned cur, link;
+  int at, end;
+};
+
+__device__ __forceinline__ TapeReader tape_reader(unsigned gi, uint4 head) {
+  return TapeReader{TAPE_CONTROL + 4u * gi, head.w, 0, TAPE_FIRST};
+}
+
+__device__ __forceinline__ uint4 tape_next(const Tape &T, TapeReader &r) {
+  if (r.at == r.end) {
+    r.cur = TAPE_CONTROL + 4u * T.photons + 16u * r.link;
+    r.link = T.cells[r.cur].w;
+    r.at = 0;
+    r.end = TAPE_MORE;
+  }
+  return T.cells[r.cur + 1 + r.at++];
+}
+
+// add n <= 64 launch indices to the replay's list (a wavefront, all its lanes)
+__device__ __forceinline__ void tape_leave(const Tape &T, const unsigned *left, int n) {
+  const int lane = threadIdx.x & 63;
+  unsigned at = 0;
+  if (n > 0 && lane == 0) at = atomicAdd(T.replay, (unsigned)n);
+  at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
+  if (lane < n) T.replay[1 + at + lane] = left[lane];
+}
+
+template <unsigned F>
+__global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArgs b) {
+  constexpr bool CHAN = F & F_CHAN;
+  const Tape &T = a.tape;
+  __shared__ unsigned s_left[TAPE_BLOCK / 64][128];  // a wavefront's photons for the replay, added to its list 64 at once
+  unsigned *left = s_left[threadIdx.x >> 6];
+  int n_left = 0;
+  double *sg = lds_cells;
+  for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
+  __syncthreads();
+  const int C = a.L[L_CLASSES];
+  const int *row_of = a.L + a.L[L_ROW_OF_AT];
+  const unsigned waves = gridDim.x * (TAPE_BLOCK / 64);
+  const unsigned w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+  const unsigned share = (T.photons + waves - 1) / waves;
+  unsigned cursor = min(w * share, T.photons);
+  const unsigned end = min(cursor + share, T.photons);
+  int read = 0;  // photons without a replay
+  while (cursor < end) {
+    unsigned gi = 0;
+    uint4 head = make_uint4(0u, 0u, 0u, 0u);
+    for (;;) {  // the wavefront's next photons with a deposit, one a lane
+      const bool need = head.z == 0u;
+      const unsigned long long mask = __ballot(need);
+      if (mask == 0ull || cursor >= end) break;
+      const unsigned i = cursor + (unsigned)lanes_below(mask);
+      bool leave = false;
+      if (need && i < end) {
+        gi = i;
+        head = T.cells[TAPE_CONTROL + 4u * i];
+        leave = head.z == TAPE_REPLAY;
+        read += leave ? 0 : 1;
+        if (leave) head.z = 0u;
+      }
+      cursor = min(cursor + (unsigned)__popcll(mask), end);
+      const unsigned long long lm = __ballot(leave);
+      if (leave) left[n_left + lanes_below(lm)] = gi;
+      n_left += __popcll(lm);
+      if (n_left >= 64) {
+        tape_leave(T, left, 64);
+        const int rest = n_left - 64, lane = threadIdx.x & 63;
+        if (lane < rest) left[lane] = left[64 + lane];
+        n_left = rest;
+      }
+    }
+    const int n = (int)head.z, event = (int)head.y;
+    if (n == 0) continue;
+    float total = 0.0f, lam = __uint_as_float(head.x);
+    TapeReader rd = tape_reader(gi, head);
+    for (int k = 0; k < n; ++k) {  // the cotangent-weighted deposits, summed in the walk's order
+      const uint4 r = tape_next(T, rd);
+      if (CHAN && (r.w & 3u) == TAPE_WAVELENGTH) {
+        lam = __uint_as_float(r.x);
+        continue;
+      }
+      const float q = __uint_as_float(r.y);
+      // a rounded product: the walk adds it, and so does the second pass
+      if (q != 0.0f) total += apart(q * deposit_cotangent(a, &b, event, lam, (int)(r.w >> 18), 0.0f));
+    }
+    Photon p;
+    p.lam = __uint_as_float(head.x);
+    p.mcls = -2;
+    float E = div_fast(HC, p.lam);  // the walk's quotient: a hoisted division would round another way
+    float sum = 0.0f;
+    rd = tape_reader(gi, head);
+    for (int k = 0; k < n; ++k) {
+      const uint4 r = tape_next(T, rd);
+      const float len = __uint_as_float(r.x), q = __uint_as_float(r.y), aux = __uint_as_float(r.z);
+      const int type = (int)(r.w & 3u), o = (int)(r.w >> 2 & 7u), pair = (int)(r.w >> 6 & 4095u);
+      if (CHAN && type == TAPE_WAVELENGTH) {
+        p.lam = len;
+        E = div_fast(HC, len);
+        p.mcls = -2;
+        continue;
+      }
+      if (p.mcls != pair / C) {  // the rates' derivatives, as medium_cache has them
+        p.mcls = pair / C;
+        p.da = p.dr = p.dm = p.dw = RateD{-1, -1, 0.0f, 0.0f};
+        const int m = class_medium(a, p.mcls);
+        if (m >= 0) {
+          const int *M = a.L + a.L[L_MEDIA_AT] + MEDIUM_WORDS * m;
+          if (!(M[8] & MED_OPAQUE)) {
+            if (M[5] > 0) p.da = rate_d(a.P, b.slots, M[4], M[5], E);
+            if (M[7] > 0) p.dr = rate_d(a.P, b.slots, M[6], M[7], E);
+            if (CHAN && (M[8] & MED_WLS)) p.dw = rate_d(a.P, b.slots, M[9], M[10], E);
+          }
+        }
+      }
+      const int *R = a.L + a.L[L_ROWS_AT] + ROW_WORDS * max(row_of[pair], 0);
+      if (q != 0.0f) {
+        const float D = apart(q * deposit_cotangent(a, &b, event, p.lam, (int)(r.w >> 18), 0.0f));
+        if (D != 0.0f) {
+          rates_add<CHAN>(sg, p, -len, -len, -len, -len, D);
+          float dsh[N_COL], ddet[N_COL];
+          surface_dlogs(R, a.P, E, -1, dsh, ddet);
+          add_columns(sg, R, a.P, b.slots, E, ddet, D);
+          sum += D;
+        }
+      }
+      const float ahead = total - sum;
+      if (ahead == 0.0f || type == TAPE_DEPOSIT) continue;
+      if (type == TAPE_SCATTER) {
+        const float kc = aux > 0.0f ? div_ieee(1.0f, aux) : 0.0f;
+        rates_add<CHAN>(sg, p, -len, (o == 0 ? kc : 0.0f) - len, (o == 1 ? kc : 0.0f) - len,
+                        (o == 2 ? kc : 0.0f) - len, ahead);
+        continue;
+      }
+      rates_add<CHAN>(sg, p, -len, -len, -len, -len, ahead);
+      if (!(r.w >> 5 & 1u)) {
+        float dsh[N_COL], ddet[N_COL];
+        surface_dlogs(R, a.P, E, o, dsh, ddet);
+        add_columns(sg, R, a.P, b.slots, E, dsh, ahead);
+      }
+      if (o == GLOSSY) {
+        const bool glisur = R[1] & FLAG_GLISUR;
+        const int col = glisur ? COL_POLISH : COL_SIGMA;
+        const float sgn = glisur ? -1.0f : 1.0f;
+        const TabD t = tab_d(a.P, b.slots, R[2 + 2 * col], R[3 + 2 * col], E);
+        grad_add(sg, t.s0, sgn * aux * t.w0 * ahead);
+        grad_add(sg, t.s1, sgn * aux * t.w1 * ahead);
+      }
+    }
+  }
+  tape_leave(T, left, n_left);
+  const float photons = wave_sum((float)read);
+  if ((threadIdx.x & 63) == 0 && photons != 0.0f) unsafeAtomicAdd(a.health + LH_H_PHOTONS, (double)photons);
+  __syncthreads();
+  for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x)
+    if (sg[i] != 0.0) unsafeAtomicAdd(b.grad + i, sg[i]);
 }
 
 }  // namespace lh
@@ -1338,6 +1563,8 @@ struct lh_model_s {
   float *ut = nullptr;  // the unified facet tables on the device
   int cus = 0, lds_per_cu = 0, lds_per_block = 0;
   bool has_chan = false;   // a medium has a Mie or WLS channel
+  bool has_mie = false;    // ... a Mie channel
+  bool has_facets = false;  // a surface row may draw a facet path
   bool has_torus = false;  // a CSG leaf is a torus (the kernels with the torus root isolation)
   // the last launch's shape: grid blocks, blocks per CU, LDS bytes per block, tallies in LDS, nodes in LDS, the
   // LDS budget per block, the CU's LDS, the kernel's feature bits
@@ -1744,8 +1971,15 @@ LH_API int lh_model_create(const lh_geometry *G, const int32_t *layout, int32_t 
       for (int c = 0; c < N_COL; ++c) need = std::max(need, (long long)R[2 + 2 * c] + 2LL * R[3 + 2 * c]);
     }
     m->values_needed = need;
-    for (int mi = 0; mi < layout[1]; ++mi)
-      if (layout[layout[6] + MEDIUM_WORDS * mi + 8] & (MED_WLS | MED_MIE)) m->has_chan = true;
+    for (int mi = 0; mi < layout[1]; ++mi) {
+      const int32_t flags = layout[layout[6] + MEDIUM_WORDS * mi + 8];
+      if (flags & (MED_WLS | MED_MIE)) m->has_chan = true;
+      if (flags & MED_MIE) m->has_mie = true;
+    }
+    for (int r = 0; r < layout[L_ROWS]; ++r) {
+      const int32_t *R = layout + layout[L_ROWS_AT] + ROW_WORDS * r;
+      if ((R[1] >> 8 >> GLOSSY) & 1) m->has_facets = true;
+    }
   }
   m->n_media = layout[1];
   m->layout_host.assign(layout, layout + layout_words);
@@ -1994,6 +2228,42 @@ static int fill_args(lh_model m, Args &a, const float *values, const float *ref,
   a.jclear = m->jclear;
   a.left_at = m->left_at;
   a.born_at = m->born_at;
+  a.tape = Tape{nullptr, nullptr, 0u, 0u};
+  a.replay = nullptr;
+  return LH_OK;
+}
+
+// The tape of a launch of `total` photons (tape.h): the bytes it takes, 0 where the launch has none.  Measured, the
+// forward + adjoint: the tank's 2^23 photons 8.19 ms with every photon replayed, 6.64 from the tape (the walk that
+// writes it takes as long as the forward; its reader 0.9 of 6.1 ns a photon); 256 sources, 5.4e7 photons, 46.0 -> 37.6;
+// the argon box, 2^18 photons, 435 -> 189 (the forward writes it: one walk of the longest path, not three).  It holds
+// the paths of a plain run, or of one with a WLS channel: reference values, Mie lobes, the diffusion jump, deposits at the
+// emission, acceptance angles, time histograms, torus roots and the reach bound leave it to the replay.  Up to 2^26
+// photons: their first chunks are 4 GiB.  The pool is 64 bytes a photon beside the wavefronts' hands (the tank's mean
+// is 15), and where a channel can shift light into a slab it is caught in, 8 KiB, up to 2 GiB (the argon box takes 4.3)
+constexpr long long TAPE_MAX_PHOTONS = 1LL << 26;
+
+static long long tape_bytes(lh_model m, const lh_controls *ctl, bool has_ref, long long total) {
+  const bool reach = m->g.n_rnode >= 0 && ctl && ctl->reach_bound;
+  if (has_ref || m->has_mie || m->NT > 0 || m->has_torus || reach || m->born_at || m->Kt > 1 || (ctl && ctl->jump) ||
+      m->layout_host[L_CLASSES] > TAPE_MAX_CLASSES || m->S > TAPE_MAX_SENSORS || total < 1 || total > TAPE_MAX_PHOTONS)
+    return 0;
+  const long long hands = 16LL * m->cus * TAPE_GRAB * 256;
+  const long long more = m->has_chan ? std::min(total * 8192, 2LL << 30) : total * 64;
+  return 16 * (long long)TAPE_CONTROL + total * 64 + (hands + more) / 256 * 256 + (total + 4) / 4 * 16;
+}
+
+// the tape at `cells` for a launch of `total` photons
+static int place_tape(lh_model m, const lh_controls *ctl, bool has_ref, long long total, void *cells, int64_t bytes,
+                      Tape &t) {
+  const long long need = tape_bytes(m, ctl, has_ref, total);
+  if (!cells || need == 0) return fail(LH_ERR_ARG, "a tape for a launch that takes none (lh_tape_size)");
+  if (bytes < need) return fail(LH_ERR_ARG, "a tape of fewer bytes than lh_tape_size");
+  if ((uintptr_t)cells % 16) return fail(LH_ERR_ARG, "a tape not aligned to 16 bytes");
+  t.cells = (uint4 *)cells;
+  t.photons = (unsigned)total;
+  t.pool = (unsigned)((need / 16 - TAPE_CONTROL - 4 * total - (total + 4) / 4) / 16);
+  t.replay = (unsigned *)(t.cells + TAPE_CONTROL + 4 * total + 16 * (long long)t.pool);
   return LH_OK;
 }
 
@@ -2007,14 +2277,19 @@ static const void *kernel_f(bool adj) {
 // the reach bound where the model has its boxes and the controls allow it; not compiled with the torus roots
 static unsigned features_of(lh_model m, const Args &a, bool adj) {
   return (a.has_ref ? F_REF : 0u) | (m->has_chan ? F_CHAN : 0u) | (!adj && m->NT > 0 ? F_TIME : 0u) |
+         (!adj && a.tape.cells ? F_TAPE : 0u) |
          (m->has_torus ? F_TORUS : 0u) | (m->g.n_rnode >= 0 && a.reach_on && !m->has_torus ? F_REACH : 0u);
 }
 
-// every feature set a launch can take: any of the first five bits, and the reach bound without the torus roots
+// every feature set a launch can take: any of the first five bits, the reach bound without the torus roots, and the
+// tape of a forward with neither reference values, time histogram, torus roots nor reach bound
 #define LH_FEATURES(X)                                                                                         \
   X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20) \
       X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31) X(32) X(33) X(34) X(35) X(36) X(37) X(38)  \
-      X(39) X(40) X(41) X(42) X(43) X(44) X(45) X(46) X(47)
+      X(39) X(40) X(41) X(42) X(43) X(44) X(45) X(46) X(47) X(64) X(66) X(72) X(74) X(192) X(194) X(200) X(202)
+
+
+
 
 // the workgroup size of a launch's kernel
 static int block_for(bool /* adjoint or forward */, unsigned /* features */) { return BLOCK; }
@@ -2144,7 +2419,14 @@ static void claim_schedule(Args &a, const lh_controls *ctl, int grid, int block,
   }
   a.first_chunk = first;
   a.dyn_at = std::min(a.total, waves * first);
-  if (a.dyn_at < a.total) hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue);
+  if ((a.dyn_at < a.total && !a.replay) || a.tape.cells)
+    hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue, a.tape.cells ? &a.tape.cells[0].x : nullptr);
+}
+
+// the adjoint's LDS: the gradient slots, then the nodes and tables
+static size_t adjoint_lds(lh_model m, Args &a, const AdjArgs &b, const lh_controls *ctl) {
+  const unsigned f = features_of(m, a, true);
+  return place_lds(m, a, kernel_of(true, f), block_for(true, f), (size_t)b.n_grad * sizeof(double), false, ctl);
 }
 
 static void launch_adjoint(lh_model m, Args &a, const AdjArgs &b, const lh_controls *ctl, size_t bytes,
@@ -2160,9 +2442,10 @@ static void launch_adjoint(lh_model m, Args &a, const AdjArgs &b, const lh_contr
 }
 
 // the forward launch: the BVH nodes and the block's tallies in LDS as they fit
-static void launch_trace(lh_model m, Args &a, int n_events, const lh_controls *ctl, hipStream_t st) {
+static void launch_trace(lh_model m, Args &a, int n_events, const lh_controls *ctl, hipStream_t st,
+                         unsigned extra = 0u) {
   const long long cells = (long long)n_events * m->tally_stride;
-  const unsigned f = features_of(m, a, false);
+  const unsigned f = features_of(m, a, false) | extra;
   const void *fn = kernel_of(false, f);
   const size_t bytes =
       place_lds(m, a, fn, block_for(false, f), cells <= LDS_TALLY_CELLS ? (size_t)cells * sizeof(double) : 0,
@@ -2178,6 +2461,29 @@ static void launch_trace(lh_model m, Args &a, int n_events, const lh_controls *c
   launch_kernel(false, fk, dim3(grid), bytes, st, a, AdjArgs{}, n_lds);
 }
 
+// the adjoint with a tape: where the model has facet paths the walk that writes it (no tallies), then the tape's reader
+// and the replay of the photons it lists.  The reader: blocks of 256 with the gradient slots in LDS; up to 8 a CU, a
+// wavefront per 64 photons at least
+static void launch_adjoint_tape(lh_model m, Args &a, const AdjArgs &b, const lh_controls *ctl, const Tape &t,
+                                hipStream_t st) {
+  Args r = a;
+  r.tape = t;
+  if (m->has_facets) {
+    Args w = r;
+    launch_trace(m, w, 0, ctl, st, F_PATH);
+  }
+  const long long want = (a.total + TAPE_BLOCK - 1) / TAPE_BLOCK;
+  const int grid = (int)std::max<long long>(1, std::min<long long>(want, (long long)m->cus * 8));
+  const size_t cells = (size_t)b.n_grad * sizeof(double);
+  hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue, t.replay);
+  if (m->has_chan)
+    hipLaunchKernelGGL(tape_adjoint_kernel<F_CHAN>, dim3(grid), dim3(TAPE_BLOCK), cells, st, r, b);
+  else
+    hipLaunchKernelGGL(tape_adjoint_kernel<0u>, dim3(grid), dim3(TAPE_BLOCK), cells, st, r, b);
+  a.replay = t.replay;
+  launch_adjoint(m, a, b, ctl, adjoint_lds(m, a, b, ctl), st);
+}
+
 // a launch on `st` after one on another stream: the model's device sources and work-queue counter are rewritten by
 // this launch, so `st` first waits for the previous launch's end (a no-op on the same stream)
 static int after_previous_launch(lh_model m, hipStream_t st) {
@@ -2185,9 +2491,9 @@ static int after_previous_launch(lh_model m, hipStream_t st) {
   return LH_OK;
 }
 
-LH_API int lh_trace(lh_model m, const float *values, const float *ref, int64_t n_values, const lh_source *sources,
-                    int32_t n_sources, uint64_t seed, const lh_controls *ctl, double *tally, int32_t n_events,
-                    double *health, void *stream) {
+static int trace_call(lh_model m, const float *values, const float *ref, int64_t n_values, const lh_source *sources,
+                      int32_t n_sources, uint64_t seed, const lh_controls *ctl, double *tally, int32_t n_events,
+                      double *health, void *tape, int64_t tape_size, void *stream) {
   if (!m) return fail(LH_ERR_ARG, "lh_trace: null model");
   if (n_values < m->values_needed) return fail(LH_ERR_ARG, "lh_trace: fewer packed values than the layout reads");
   for (int i = 0; i < n_sources && sources; ++i)
@@ -2203,6 +2509,8 @@ LH_API int lh_trace(lh_model m, const float *values, const float *ref, int64_t n
   if (rc) return rc;
   a.nsrc = n_sources;
   a.total = total;
+  if (tape && (rc = place_tape(m, ctl, a.has_ref != 0, total, tape, tape_size, a.tape))) return rc;
+  if (m->has_facets) a.tape.cells = nullptr;
   const int slot = (int)(m->launches % TIME_RING);
   HIP_TRY(hipEventRecord(m->ev0[slot], st));
   launch_trace(m, a, n_events, ctl, st);
@@ -2210,6 +2518,28 @@ LH_API int lh_trace(lh_model m, const float *values, const float *ref, int64_t n
   HIP_TRY(hipEventRecord(m->ev1[slot], st));
   ++m->launches;
   return LH_OK;
+}
+
+LH_API int lh_trace(lh_model m, const float *values, const float *ref, int64_t n_values, const lh_source *sources,
+                    int32_t n_sources, uint64_t seed, const lh_controls *ctl, double *tally, int32_t n_events,
+                    double *health, void *stream) {
+  return trace_call(m, values, ref, n_values, sources, n_sources, seed, ctl, tally, n_events, health, nullptr, 0, stream);
+}
+
+LH_API int lh_tape_size(lh_model m, const lh_controls *ctl, int32_t has_ref, int64_t photons, int64_t *bytes,
+                        int32_t *by_adjoint) {
+  if (!m || !bytes || !by_adjoint) return fail(LH_ERR_ARG, "lh_tape_size: null model or output");
+  *bytes = tape_bytes(m, ctl, has_ref != 0, photons);
+  *by_adjoint = m->has_facets ? 1 : 0;
+  return LH_OK;
+}
+
+LH_API int lh_trace_tape(lh_model m, const float *values, int64_t n_values, const lh_source *sources, int32_t n_sources,
+                         uint64_t seed, const lh_controls *ctl, double *tally, int32_t n_events, double *health,
+                         void *tape, int64_t tape_size, void *stream) {
+  if (!tape) return fail(LH_ERR_ARG, "lh_trace_tape: null tape");
+  return trace_call(m, values, nullptr, n_values, sources, n_sources, seed, ctl, tally, n_events, health, tape,
+                    tape_size, stream);
 }
 
 // the staged sources' end offsets (a prefix sum of their photon counts) and a cleared work queue, for
@@ -2266,10 +2596,10 @@ LH_API int lh_trace_static(lh_model m, const float *values, const float *ref, in
   return LH_OK;
 }
 
-LH_API int lh_adjoint(lh_model m, const float *values, const float *ref, int64_t n_values, const int32_t *slots,
-                      const lh_source *sources, int32_t n_sources, uint64_t seed, const lh_controls *ctl,
-                      const double *cot, int32_t n_events, double *grad, int32_t n_grad, double *health,
-                      void *stream) {
+static int adjoint_call(lh_model m, const float *values, const float *ref, int64_t n_values, const int32_t *slots,
+                        const lh_source *sources, int32_t n_sources, uint64_t seed, const lh_controls *ctl,
+                        const double *cot, int32_t n_events, double *grad, int32_t n_grad, double *health, void *tape,
+                        int64_t tape_size, void *stream) {
   if (!m) return fail(LH_ERR_ARG, "lh_adjoint: null model");
   if (n_values < m->values_needed) return fail(LH_ERR_ARG, "lh_adjoint: fewer packed values than the layout reads");
   if (!slots || !cot || !grad) return fail(LH_ERR_ARG, "lh_adjoint: null slots, cotangent or gradient");
@@ -2295,15 +2625,35 @@ LH_API int lh_adjoint(lh_model m, const float *values, const float *ref, int64_t
   a.nsrc = n_sources;
   a.total = total;
   AdjArgs b{cot, slots, grad, n_grad};
+  Tape t{nullptr, nullptr, 0u, 0u};
+  if (tape && (rc = place_tape(m, ctl, a.has_ref != 0, total, tape, tape_size, t))) return rc;
   const int slot = (int)(m->launches % TIME_RING);
   HIP_TRY(hipEventRecord(m->ev0[slot], st));
-  const size_t bytes = place_lds(m, a, kernel_of(true, features_of(m, a, true)), block_for(true, features_of(m, a, true)),
-                                 (size_t)n_grad * sizeof(double), false, ctl);
-  launch_adjoint(m, a, b, ctl, bytes, st);
+  if (tape)
+    launch_adjoint_tape(m, a, b, ctl, t, st);
+  else
+    launch_adjoint(m, a, b, ctl, adjoint_lds(m, a, b, ctl), st);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(m->ev1[slot], st));
   ++m->launches;
   return LH_OK;
+}
+
+LH_API int lh_adjoint(lh_model m, const float *values, const float *ref, int64_t n_values, const int32_t *slots,
+                      const lh_source *sources, int32_t n_sources, uint64_t seed, const lh_controls *ctl,
+                      const double *cot, int32_t n_events, double *grad, int32_t n_grad, double *health,
+                      void *stream) {
+  return adjoint_call(m, values, ref, n_values, slots, sources, n_sources, seed, ctl, cot, n_events, grad, n_grad,
+                      health, nullptr, 0, stream);
+}
+
+LH_API int lh_adjoint_tape(lh_model m, const float *values, int64_t n_values, const int32_t *slots,
+                           const lh_source *sources, int32_t n_sources, uint64_t seed, const lh_controls *ctl,
+                           const double *cot, int32_t n_events, double *grad, int32_t n_grad, double *health,
+                           void *tape, int64_t tape_size, void *stream) {
+  if (!tape) return fail(LH_ERR_ARG, "lh_adjoint_tape: null tape");
+  return adjoint_call(m, values, nullptr, n_values, slots, sources, n_sources, seed, ctl, cot, n_events, grad, n_grad,
+                      health, tape, tape_size, stream);
 }
 
 // a staged batch (lh_batch_create): its own sources, work queue and checked gradient slots
@@ -2365,8 +2715,9 @@ LH_API int lh_batch_destroy(lh_batch b) {
   return LH_OK;
 }
 
-LH_API int lh_batch_trace(lh_batch b, const float *values, const float *ref, int64_t n_values, uint64_t seed,
-                          const lh_controls *ctl, double *tally, int32_t n_events, double *health, void *stream) {
+static int batch_trace_call(lh_batch b, const float *values, const float *ref, int64_t n_values, uint64_t seed,
+                            const lh_controls *ctl, double *tally, int32_t n_events, double *health, void *tape,
+                            int64_t tape_size, void *stream) {
   if (!b) return fail(LH_ERR_ARG, "lh_batch_trace: null batch");
   lh_model m = b->m;
   if (n_values < m->values_needed) return fail(LH_ERR_ARG, "lh_batch_trace: fewer packed values than the layout reads");
@@ -2380,14 +2731,28 @@ LH_API int lh_batch_trace(lh_batch b, const float *values, const float *ref, int
   a.nsrc = b->nsrc;
   a.total = b->total;
   a.queue = b->queue;
+  if (tape && (rc = place_tape(m, ctl, a.has_ref != 0, b->total, tape, tape_size, a.tape))) return rc;
+  if (m->has_facets) a.tape.cells = nullptr;
   launch_trace(m, a, n_events, ctl, st);
   HIP_TRY(hipGetLastError());
   return LH_OK;
 }
 
-LH_API int lh_batch_adjoint(lh_batch b, const float *values, const float *ref, int64_t n_values, uint64_t seed,
-                            const lh_controls *ctl, const double *cot, int32_t n_events, double *grad, int32_t n_grad,
-                            double *health, void *stream) {
+LH_API int lh_batch_trace(lh_batch b, const float *values, const float *ref, int64_t n_values, uint64_t seed,
+                          const lh_controls *ctl, double *tally, int32_t n_events, double *health, void *stream) {
+  return batch_trace_call(b, values, ref, n_values, seed, ctl, tally, n_events, health, nullptr, 0, stream);
+}
+
+LH_API int lh_batch_trace_tape(lh_batch b, const float *values, int64_t n_values, uint64_t seed, const lh_controls *ctl,
+                               double *tally, int32_t n_events, double *health, void *tape, int64_t tape_size,
+                               void *stream) {
+  if (!tape) return fail(LH_ERR_ARG, "lh_batch_trace_tape: null tape");
+  return batch_trace_call(b, values, nullptr, n_values, seed, ctl, tally, n_events, health, tape, tape_size, stream);
+}
+
+static int batch_adjoint_call(lh_batch b, const float *values, const float *ref, int64_t n_values, uint64_t seed,
+                              const lh_controls *ctl, const double *cot, int32_t n_events, double *grad, int32_t n_grad,
+                              double *health, void *tape, int64_t tape_size, void *stream) {
   if (!b) return fail(LH_ERR_ARG, "lh_batch_adjoint: null batch");
   lh_model m = b->m;
   if (!b->slots) return fail(LH_ERR_ARG, "lh_batch_adjoint: the batch was created without gradient slots");
@@ -2405,11 +2770,29 @@ LH_API int lh_batch_adjoint(lh_batch b, const float *values, const float *ref, i
   a.total = b->total;
   a.queue = b->queue;
   AdjArgs g{cot, b->slots, grad, n_grad};
-  const size_t bytes = place_lds(m, a, kernel_of(true, features_of(m, a, true)), block_for(true, features_of(m, a, true)),
-                                 (size_t)n_grad * sizeof(double), false, ctl);
-  launch_adjoint(m, a, g, ctl, bytes, st);
+  Tape t{nullptr, nullptr, 0u, 0u};
+  if (tape && (rc = place_tape(m, ctl, a.has_ref != 0, b->total, tape, tape_size, t))) return rc;
+  if (tape)
+    launch_adjoint_tape(m, a, g, ctl, t, st);
+  else
+    launch_adjoint(m, a, g, ctl, adjoint_lds(m, a, g, ctl), st);
   HIP_TRY(hipGetLastError());
   return LH_OK;
+}
+
+LH_API int lh_batch_adjoint(lh_batch b, const float *values, const float *ref, int64_t n_values, uint64_t seed,
+                            const lh_controls *ctl, const double *cot, int32_t n_events, double *grad, int32_t n_grad,
+                            double *health, void *stream) {
+  return batch_adjoint_call(b, values, ref, n_values, seed, ctl, cot, n_events, grad, n_grad, health, nullptr, 0,
+                            stream);
+}
+
+LH_API int lh_batch_adjoint_tape(lh_batch b, const float *values, int64_t n_values, uint64_t seed,
+                                 const lh_controls *ctl, const double *cot, int32_t n_events, double *grad,
+                                 int32_t n_grad, double *health, void *tape, int64_t tape_size, void *stream) {
+  if (!tape) return fail(LH_ERR_ARG, "lh_batch_adjoint_tape: null tape");
+  return batch_adjoint_call(b, values, nullptr, n_values, seed, ctl, cot, n_events, grad, n_grad, health, tape,
+                            tape_size, stream);
 }
 
 LH_API int lh_query(lh_model m, int32_t n, const float *x_dev, const float *d_dev, const int32_t *vol_dev,
