@@ -712,10 +712,11 @@ __device__ inline Cross query_t(const Geo &g, float3 x, float3 d, int vol, int l
     const float3 xp = fma3(best.t + step, d, x);
     int v2 = best.vol_after;
     if (best.own) {
+      const int near = g.vinfo[vol].x;
       float3 xl, dl;
-      to_local(g, best.vol_after, xp, d, xl, dl);
-      if (!solid_inside<TOR>(g, g.vkind[best.vol_after], xl)) v2 = locate<TOR>(g, xp);
-      else if (g.vinfo[vol].x & 1) v2 = locate<TOR>(g, xp, best.vol_after);
+      if (!(near & 2)) to_local(g, best.vol_after, xp, d, xl, dl);
+      if (!(near & 2) && !solid_inside<TOR>(g, g.vkind[best.vol_after], xl)) v2 = locate<TOR>(g, xp);
+      else if (near & 1) v2 = locate<TOR>(g, xp, best.vol_after);
     } else {
       const int2 gr = g.vgrp[best.vol_after];
       if (gr.x < gr.y) v2 = locate<TOR>(g, xp, best.vol_after);
