@@ -79,9 +79,16 @@ constexpr unsigned F_ADJ_MASK = F_REF | F_CHAN | F_GNODES | F_TORUS | F_REACH;
 #endif
 #define LH_OCC_FWD(F) __attribute__((amdgpu_waves_per_eu(LH_WAVES_PER_EU)))
 
+// where the layout's tables begin and its class count: of the launch's arguments, not read from the layout's header step
+// after step (each a load before the load it is for: argon light map 159 -> 155 ms, tank event of 2^24 photons 5.07 -> 5.03)
+struct LayoutAt {
+  int media, class_medium, row_of, rows, classes;
+};
+
 struct Args {
   Geo g;
   const int *__restrict__ L;
+  LayoutAt at;
   const float *__restrict__ P;
   const float *__restrict__ Pr;
   int has_ref;
@@ -182,7 +189,7 @@ __device__ __forceinline__ float pick6(const float a[6], int o) {
 }
 
 __device__ __forceinline__ int class_medium(const Args &a, int cls) {
-  return cls < 0 ? -1 : a.L[a.L[L_CLASS_MEDIUM_AT] + cls];
+  return cls < 0 ? -1 : a.L[a.at.class_medium + cls];
 }
 
 
@@ -344,7 +351,7 @@ __device__ inline bool emit(const Args &a, long long gi, Photon &p, Acc &acc) {
   p.er = p.ei = mk3(0.f, 0.f, 0.f);
   p.event = S.event;
   if (S.kind == LH_SRC_CHERENKOV) {
-    const int *M = a.L + a.L[L_MEDIA_AT] + MEDIUM_WORDS * S.medium;
+    const int *M = a.L + a.at.media + MEDIUM_WORDS * S.medium;
     const float e_lo = a.P[M[0]], e_hi = a.P[M[0] + M[1] - 1];
     const float lam_min = HC / e_hi, lam_max = HC / e_lo;
     const float zq = 1.0f / lam_min - 1.0f / lam_max;
@@ -584,8 +591,8 @@ __device__ inline void medium_cache(const Args &a, Photon &p, const AdjArgs *b) 
   constexpr bool REF = F & F_REF, CHAN = F & F_CHAN;
   if (p.mcls == p.cls) return;
   const int m = class_medium(a, p.cls);
-  p.ml = medium_at(a.L, a.P, m, p.lam);
-  if (REF) p.mr = medium_at(a.L, a.Pr, m, p.lam);
+  p.ml = medium_at(a.L + a.at.media, a.P, m, p.lam);
+  if (REF) p.mr = medium_at(a.L + a.at.media, a.Pr, m, p.lam);
   p.mcls = p.cls;
   if (ADJ) {
     p.da = RateD{-1, -1, 0.0f, 0.0f};
@@ -593,7 +600,7 @@ __device__ inline void medium_cache(const Args &a, Photon &p, const AdjArgs *b) 
     p.dm = RateD{-1, -1, 0.0f, 0.0f};
     p.dw = RateD{-1, -1, 0.0f, 0.0f};
     if (m >= 0) {
-      const int *M = a.L + a.L[L_MEDIA_AT] + MEDIUM_WORDS * m;
+      const int *M = a.L + a.at.media + MEDIUM_WORDS * m;
       if (!(M[8] & MED_OPAQUE)) {
         const float E = HC / p.lam;
         if (M[5] > 0) p.da = rate_d(a.P, b->slots, M[4], M[5], E);
@@ -723,7 +730,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
   if (a.born_at && p.vertex == 0) {  // emitted inside a sensor volume that counts by volume (step.py:574-612 `_born`)
     const int br = a.L[a.born_at + p.cls], sensor = g.vinfo[p.vol].w;
     if (br >= 0 && sensor >= 0) {  // the entry's detected share, deposited at the emission; the photon ends there
-      const SurfEval se = surface_eval(a.L, a.P, br, p.lam, p.d, mul3(-1.0f, p.d), 1.0f, 1.0f, er0, ei0);
+      const SurfEval se = surface_eval(a.L + a.at.rows, a.P, br, p.lam, p.d, mul3(-1.0f, p.d), 1.0f, 1.0f, er0, ei0);
       const float dep_q = p.w * se.detect;
       const float theta = a.Kt > 1 ? cathode_theta(g, p.vol, p.x) : 0.0f;
       if (!ADJ) {
@@ -735,7 +742,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
           p.hasdep = true;
           if (p.pass == 1) {
             float dsh[N_COL], ddet[N_COL];
-            const int *Rw = a.L + a.L[L_ROWS_AT] + ROW_WORDS * br;
+            const int *Rw = a.L + a.at.rows + ROW_WORDS * br;
             surface_dlogs(Rw, a.P, HC / p.lam, -1, dsh, ddet);
             add_columns(sg, Rw, a.P, b->slots, HC / p.lam, ddet, D);
           }
@@ -767,7 +774,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
   const bool zero = dist <= ZERO_STEP_BANDS * b0;
   const int cb = p.cls;
   const int ca = hit ? g.vinfo[cr.vol_after].z : -1;
-  int row = hit ? a.L[a.L[L_ROW_OF_AT] + cb * a.L[L_CLASSES] + ca] : -1;
+  int row = hit ? a.L[a.at.row_of + cb * a.at.classes + ca] : -1;
   // a crossing no surface joins, of zero length or between two volumes of one class (the same medium and surfaces,
   // which the reference's navigator does not stop at: lookup.py:26-31): a straight pass
   const bool cont = hit && (zero || ca == cb) && row < 0;
@@ -779,7 +786,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
   if (TAPE) {  // the step's record (tape.h), so far a deposit's
     p.rec.len = apart(dist);
     p.rec.free = p.rec.dep = p.rec.aux = 0.0f;
-    p.rec.code = tape_code(TAPE_DEPOSIT, 0, cont, cb * a.L[L_CLASSES] + (ca < 0 ? 0 : ca), 0);
+    p.rec.code = tape_code(TAPE_DEPOSIT, 0, cont, cb * a.at.classes + (ca < 0 ? 0 : ca), 0);
   }
   SurfEval sl, sr;
   int o = -1;
@@ -788,19 +795,19 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
   if (at_if) {
     const int m2 = class_medium(a, ca);
     if (CHAN && p.ncls != ca) {
-      p.n2 = index_at(a.L, a.P, m2, p.lam);
+      p.n2 = index_at(a.L + a.at.media, a.P, m2, p.lam);
       p.ncls = ca;
     }
-    const float n2 = CHAN ? p.n2 : index_at(a.L, a.P, m2, p.lam);
-    sl = surface_eval(a.L, a.P, row, p.lam, p.d, cr.n, ml.n, n2, er0, ei0);
+    const float n2 = CHAN ? p.n2 : index_at(a.L + a.at.media, a.P, m2, p.lam);
+    sl = surface_eval(a.L + a.at.rows, a.P, row, p.lam, p.d, cr.n, ml.n, n2, er0, ei0);
     if (cont) {
       for (int k = 0; k < N_OUT; ++k) sl.p[k] = 0.0f;
       sl.p[STRAIGHT] = 1.0f;
       sl.detect = 0.0f;
     }
     if (REF) {
-      const float n2r = index_at(a.L, a.Pr, m2, p.lam);
-      sr = surface_eval(a.L, a.Pr, row, p.lam, p.d, cr.n, mr.n, n2r, er0, ei0);
+      const float n2r = index_at(a.L + a.at.media, a.Pr, m2, p.lam);
+      sr = surface_eval(a.L + a.at.rows, a.Pr, row, p.lam, p.d, cr.n, mr.n, n2r, er0, ei0);
       if (cont) {
         for (int k = 0; k < N_OUT; ++k) sr.p[k] = 0.0f;
         sr.p[STRAIGHT] = 1.0f;
@@ -830,7 +837,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
     // the deposit: the expected detection at the crossing (step.py:522-524)
     const float dep_q = p.w * reach_live * att * sl.detect;
     // the sensor entered, or across an exit sensor's border the region left (step.py:544-547 `_sensor_dep`)
-    const int vs = (a.left_at && a.L[a.left_at + cb * a.L[L_CLASSES] + ca]) ? p.vol : cr.vol_after;
+    const int vs = (a.left_at && a.L[a.left_at + cb * a.at.classes + ca]) ? p.vol : cr.vol_after;
     const int sensor = g.vinfo[vs].w;
     if (sensor >= 0 && !cont) {
       const float theta = a.Kt > 1 ? cathode_theta(g, vs, fma3(dist, p.d, p.x)) : 0.0f;
@@ -847,7 +854,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
           if (p.pass == 1) {  // the deposit's own factors: reach, attenuation, the detected share
             rates_add<CHAN>(sg, p, -dist, -dist, -dist, -dist, D);
             float dsh[N_COL], ddet[N_COL];
-            const int *Rw = a.L + a.L[L_ROWS_AT] + ROW_WORDS * row;
+            const int *Rw = a.L + a.at.rows + ROW_WORDS * row;
             surface_dlogs(Rw, a.P, HC / p.lam, -1, dsh, ddet);
             add_columns(sg, Rw, a.P, b->slots, HC / p.lam, ddet, D);
           }
@@ -896,7 +903,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
         dn = rayleigh_sample(er0, ei0, ul[0], ul[1], ul[2]);
       } else {  // G4OpMieHG, drawn at the reference's lobes under the cover of its forward ratio, weighted by the
                 // live mixture density over the drawn one (transport/medium.py:96-133 `channel_draw`)
-        const int *M = a.L + a.L[L_MEDIA_AT] + MEDIUM_WORDS * class_medium(a, p.cls);
+        const int *M = a.L + a.at.media + MEDIUM_WORDS * class_medium(a, p.cls);
         const MieLobe lv = mie_lobe(a.P, M), lr = REF ? mie_lobe(a.Pr, M) : lv;
         const float rc = mie_cover(lr.r);
         dn = mie_sample(p.d, lr.gf, lr.gb, rc, ul[0], ul[1], ul[2]);
@@ -941,7 +948,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
     } else {  // a wavelength shifter (G4OpWLS): re-emitted isotropic, unpolarised, after the record's delay
       float ur[4];
       rng.draw4(p.vertex, 2, ur);  // (wavelength, delay, -, -)
-      const int *M = a.L + a.L[L_MEDIA_AT] + MEDIUM_WORDS * class_medium(a, p.cls);
+      const int *M = a.L + a.at.media + MEDIUM_WORDS * class_medium(a, p.cls);
       const WlsDraw em = wls_emit(a.P, REF ? a.Pr : a.P, M, p.lam, ur[0], ur[1]);
       w_new = w_at * att_s * em.w;
       wr_new = p.wr * att_s_r * em.wr;
@@ -971,7 +978,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
     if (ok && adj_event) {  // reach, attenuation over the segment, and the drawn outcome's share
       rates_add<CHAN>(sg, p, -dist, -dist, -dist, -dist, ahead);
       float dsh[N_COL], ddet[N_COL];
-      const int *Rw = a.L + a.L[L_ROWS_AT] + ROW_WORDS * row;
+      const int *Rw = a.L + a.at.rows + ROW_WORDS * row;
       if (!cont) {
         surface_dlogs(Rw, a.P, HC / p.lam, o, dsh, ddet);
         add_columns(sg, Rw, a.P, b->slots, HC / p.lam, dsh, ahead);
@@ -989,7 +996,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
       if (o == STRAIGHT) {
         far = true;
       } else if (o == REFRACT) {
-        const float m2n = index_at(a.L, a.P, class_medium(a, ca), p.lam);
+        const float m2n = index_at(a.L + a.at.media, a.P, class_medium(a, ca), p.lam);
         dn = refract_dir(wi, n, ml.n / m2n);
         pol_recombine(er0, ei0, wi, s_axis(wi, n), sl.amps.ts, sl.amps.tp, unit3(dn));
         far = true;
@@ -1008,7 +1015,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
           // refracts too and may end beyond the surface (at the live indices, as a polished interface)
           const bool cover = sr.flags & FLAG_COVER, weigh = want_ratio || cover;
           if (sr.flags & FLAG_REFRACTS) {
-            const float n2l = index_at(a.L, a.P, class_medium(a, ca), p.lam);
+            const float n2l = index_at(a.L + a.at.media, a.P, class_medium(a, ca), p.lam);
             dn = glisur_dielectric(rng, p.vertex, sr.sigma, sl.sigma, cover, weigh, PATH || adj_event, wi, n, ml.n, n2l,
                                    er0, ei0, logw, dlogw, far);
           } else {
@@ -1025,7 +1032,7 @@ __device__ inline bool step(const Args &a, Photon &p, Acc &acc, const AdjArgs *b
         if (adj_event) {  // the live log density's derivative in the width: sigma_alpha, or -d/dr for polish
           const int col = glisur ? COL_POLISH : COL_SIGMA;
           const float sgn = glisur ? -1.0f : 1.0f;
-          const int *Rw = a.L + a.L[L_ROWS_AT] + ROW_WORDS * row;
+          const int *Rw = a.L + a.at.rows + ROW_WORDS * row;
           const TabD t = tab_d(a.P, b->slots, Rw[2 + 2 * col], Rw[3 + 2 * col], HC / p.lam);
           grad_add(sg, t.s0, sgn * dlogw * t.w0 * ahead);
           grad_add(sg, t.s1, sgn * dlogw * t.w1 * ahead);
@@ -1407,8 +1414,8 @@ __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArg
   double *sg = lds_cells;
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
   __syncthreads();
-  const int C = a.L[L_CLASSES];
-  const int *row_of = a.L + a.L[L_ROW_OF_AT];
+  const int C = a.at.classes;
+  const int *row_of = a.L + a.at.row_of;
   const unsigned waves = gridDim.x * (TAPE_BLOCK / 64);
   const unsigned w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
   const unsigned share = (T.photons + waves - 1) / waves;
@@ -1477,7 +1484,7 @@ __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArg
         p.da = p.dr = p.dm = p.dw = RateD{-1, -1, 0.0f, 0.0f};
         const int m = class_medium(a, p.mcls);
         if (m >= 0) {
-          const int *M = a.L + a.L[L_MEDIA_AT] + MEDIUM_WORDS * m;
+          const int *M = a.L + a.at.media + MEDIUM_WORDS * m;
           if (!(M[8] & MED_OPAQUE)) {
             if (M[5] > 0) p.da = rate_d(a.P, b.slots, M[4], M[5], E);
             if (M[7] > 0) p.dr = rate_d(a.P, b.slots, M[6], M[7], E);
@@ -1485,7 +1492,7 @@ __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArg
           }
         }
       }
-      const int *R = a.L + a.L[L_ROWS_AT] + ROW_WORDS * max(row_of[pair], 0);
+      const int *R = a.L + a.at.rows + ROW_WORDS * max(row_of[pair], 0);
       if (q != 0.0f) {
         const float D = apart(q * deposit_cotangent(a, &b, event, p.lam, (int)(r.w >> 18), 0.0f));
         if (D != 0.0f) {
@@ -2238,6 +2245,8 @@ static int fill_args(lh_model m, Args &a, const float *values, const float *ref,
   if (!tally || !health) return fail(LH_ERR_ARG, "null tally or health");
   a.g = m->g;
   a.L = m->layout;
+  a.at = LayoutAt{m->layout_host[L_MEDIA_AT], m->layout_host[L_CLASS_MEDIUM_AT], m->layout_host[L_ROW_OF_AT],
+                  m->layout_host[L_ROWS_AT], m->layout_host[L_CLASSES]};
   a.P = values;
   a.Pr = ref ? ref : values;
   a.has_ref = (ref && ref != values) ? 1 : 0;

@@ -78,10 +78,10 @@ struct MediumAt {
   float n, ng, mu_abs, mu_ray, mu_mie, mu_wls;  // the event channels' rates in Geant4's order: Rayleigh, Mie, WLS
 };
 
-__device__ inline MediumAt medium_at(const int *__restrict__ L, const float *__restrict__ P, int m, float lam) {
+__device__ inline MediumAt medium_at(const int *__restrict__ media, const float *__restrict__ P, int m, float lam) {
   MediumAt r{1.0f, 1.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   if (m < 0) return r;
-  const int *M = L + L[L_MEDIA_AT] + MEDIUM_WORDS * m;
+  const int *M = media + MEDIUM_WORDS * m;
   if (M[8] & MED_OPAQUE) return r;
   const float E = HC / lam;
   const TabPos pn = tab_pos(P, M[0], M[1], E);
@@ -199,9 +199,9 @@ __device__ inline WlsDraw wls_emit(const float *__restrict__ P, const float *__r
   return r;
 }
 
-__device__ __forceinline__ float index_at(const int *__restrict__ L, const float *__restrict__ P, int m, float lam) {
+__device__ __forceinline__ float index_at(const int *__restrict__ media, const float *__restrict__ P, int m, float lam) {
   if (m < 0) return 1.0f;
-  const int *M = L + L[L_MEDIA_AT] + MEDIUM_WORDS * m;
+  const int *M = media + MEDIUM_WORDS * m;
   if (M[8] & MED_OPAQUE) return 1.0f;
   return tab(P, M[0], M[1], HC / lam);
 }
@@ -382,10 +382,10 @@ __device__ __forceinline__ float col_at(const int *__restrict__ R, const float *
 
 // one surface row at a crossing: Geant4's chain (types.py:211-296): r, t, a = chained_cuts(Rc, T), r split by the
 // reflection constants (or the Fresnel interface), t straight on, a detected with eff
-__device__ inline SurfEval surface_eval(const int *__restrict__ L, const float *__restrict__ P, int row, float lam,
+__device__ inline SurfEval surface_eval(const int *__restrict__ rows, const float *__restrict__ P, int row, float lam,
                                         float3 wi, float3 n, float n1, float n2, float3 er, float3 ei) {
   SurfEval s;
-  const int *R = L + L[L_ROWS_AT] + ROW_WORDS * row;
+  const int *R = rows + ROW_WORDS * row;
   const int model = R[0], flags = R[1];
   s.flags = flags;
   const RowCols col = row_cols(R, P, HC / lam);
