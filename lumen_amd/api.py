@@ -221,6 +221,16 @@ def moment_error(q2, s, n: int):
     return torch.sqrt(torch.clamp(n / (n - 1.0) * (q2 - s * s / n), min=0.0))
 
 
+def to_device(a: np.ndarray, device):
+    """Return the array on the device, copied on the current stream without waiting for it: a copy from pageable memory
+    waits for all the stream holds, the photon loop launched before it included (a call of 10^5 photons in the tank
+    then takes its host time and its kernel's one after the other)."""  # noqa: D205, D209
+    import torch
+
+    t = torch.from_numpy(np.array(a))
+    return t.pin_memory().to(device, non_blocking=True) if torch.device(device).type == "cuda" else t.to(device)
+
+
 class Engine:
     """A detector's model on the device (built once per detector and device) and its run state."""
 
@@ -335,14 +345,11 @@ class Engine:
             return None
 
     def upload(self, values: np.ndarray):
-        """Return the packed values on the device, the previous upload again when they are the same (a copy from
-        pageable memory waits for the stream; unchanged values need none)."""  # noqa: D205, D209
-        import torch
-
+        """Return the packed values on the device, the previous upload again when they are the same."""
         last = self._uploads.get(values.nbytes)
         if last is not None and np.array_equal(last[0], values):
             return last[1]
-        t = torch.as_tensor(values, device=self.device)
+        t = to_device(values, self.device)
         self._uploads[values.nbytes] = (values.copy(), t)
         return t
 
@@ -496,7 +503,7 @@ def simulate(det, source, params: Params | None = None, *, samples: int | None =
         pr = packing.pack(det, reference, edge_rows=edge_rows)
         if not np.array_equal(pr.layout, eng.layout):
             raise ValueError("simulate: the reference's structure differs from the detector's")
-        ref_values = torch.as_tensor(pr.values, device=eng.device)
+        ref_values = to_device(pr.values, eng.device)
     rows, n_ev = source_rows(det, source, samples, first_id)
     if events is not None:
         if int(events) < n_ev:
@@ -559,7 +566,7 @@ def light_of(eng, tally, health, samples, source=None, keep_events=False) -> Lig
         ev = np.arange(len(source.samples)) if source.events is None else np.asarray(source.events, np.int64)
         per_event = np.bincount(ev, weights=np.asarray(source.samples, np.float64), minlength=tally.shape[0])
         per_event = per_event[: tally.shape[0]]
-        n = torch.as_tensor(np.maximum(per_event, 2.0), dtype=torch.float64, device=tally.device)[:, None]
+        n = to_device(np.maximum(per_event, 2.0), tally.device)[:, None]
         err = torch.sqrt(torch.clamp(n / (n - 1.0) * (arr2 - arr * arr / n), min=0.0))
     else:
         err = moment_error(arr2, arr, samples)

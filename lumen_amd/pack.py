@@ -57,13 +57,10 @@ def group_index_knots(e, n):
     if k < 1:
         return e.copy(), n.copy()
     eg = np.concatenate([e[:1], 0.5 * (e[:-2] + e[1:-1]), e[-1:]])
-    ng = np.zeros(k + 1)
-    for j in range(k + 1):
-        s = min(max(j - 1, 0), k - 1)
-        slope = (n[s + 1] - n[s]) / np.log(e[s + 1] / e[s])
-        base = n[j] if j in (0, k) else 0.5 * (n[s] + n[s + 1])
-        ng[j] = max(base + slope, base)
-    return eg, ng
+    slope = np.diff(n) / np.log(e[1:] / e[:-1])  # per segment; knot j has segment j - 1's, knot 0 the first's
+    slope = np.concatenate([slope[:1], slope])
+    base = np.concatenate([n[:1], 0.5 * (n[:-2] + n[1:-1]), n[-1:]])
+    return eg, np.maximum(base + slope, base)
 
 
 def water_rayleigh(e, n):
@@ -94,14 +91,21 @@ class _Builder:
         self.n_grad = 0
         self.grad_map = []
 
+    def constant(self, v):
+        """A table of one knot and no key: a row's fixed column (most of a pack's tables)."""
+        off = len(self.vals)
+        self.vals += [0.0, v]
+        self.slots += [-1, -1]
+        return off, 1
+
     def table(self, e, v, key=None):
         e, v = np.atleast_1d(np.asarray(e, np.float64)), np.atleast_1d(np.asarray(v, np.float64))
         if e.shape != v.shape or len(e) == 0:
             raise ValueError(f"pack: table {key!r} has {len(e)} knots and {len(v)} values")
-        if len(e) > 1 and np.any(np.diff(e) <= 0):
+        if len(e) > 1 and (e[1:] - e[:-1] <= 0).any():
             raise ValueError(f"pack: table {key!r}: knots must ascend")
         off = len(self.vals)
-        self.vals += list(e) + list(v)
+        self.vals += e.tolist() + v.tolist()
         slot = -1
         if key is not None and key in self.grad:
             if self.grad[key] is None:
@@ -203,7 +207,7 @@ def pack(det: Detector, params: Params | None = None, grad_keys=(), edge_rows="s
         rows[r, 1] = row.flags() | (FLAG_EDGE if r in edge_rows else 0)
         for j, c in enumerate(COLUMNS):
             v = row.column(c)
-            rows[r, 2 + 2 * j: 4 + 2 * j] = b.value(p, v) if isinstance(v, str) else b.table([0.0], [float(v)])
+            rows[r, 2 + 2 * j: 4 + 2 * j] = b.value(p, v) if isinstance(v, str) else b.constant(float(v))
         if row.type.startswith("GLISUR") and isinstance(row.columns["polish"], str):
             pv = p[row.columns["polish"]]
             for x in np.atleast_1d(pv.value if isinstance(pv, Table) else pv):
@@ -213,25 +217,25 @@ def pack(det: Detector, params: Params | None = None, grad_keys=(), edge_rows="s
     if isinstance(q, Table):  # the charge histogram's wavelength knots (nm); QE itself is read after tracking
         qe_off, n_qe = b.table(q.energy, q.value)
     else:  # no QE table, or one QE per sensor: a single charge cell per sensor
-        qe_off, n_qe = b.table([0.0], [1.0])
+        qe_off, n_qe = b.constant(1.0)
     ce = p[det.groups[0].ce] if det.groups and getattr(det.groups[0], "ce", None) is not None else None
     if isinstance(ce, Table) and len(ce.energy) > 1:  # the charge histogram's theta knots (rad); CE read after tracking
         ce_off, n_ce = b.table(ce.energy, ce.value)
     else:
-        ce_off, n_ce = b.table([0.0], [1.0])
+        ce_off, n_ce = b.constant(1.0)
     tg = getattr(det, "time_grid", None)
     f32bits = lambda x: int(np.array([x], np.float32).view(np.int32)[0])  # noqa: E731
     L = [MAGIC, nm, nc, nr, det.n_sensors, n_qe, 0, 0, 0, 0, qe_off,
          0 if tg is None else tg.nt, 0 if tg is None else f32bits(tg.t0), 0 if tg is None else f32bits(tg.dt),
          n_ce, ce_off, 0, 0]
     L[6] = len(L)
-    L += list(med.ravel())
+    L += med.ravel().tolist()
     L[7] = len(L)
-    L += list(np.asarray(det.class_medium, np.int32))
+    L += np.asarray(det.class_medium, np.int32).tolist()
     L[8] = len(L)
-    L += list(np.asarray(det.row_of, np.int32).ravel())
+    L += np.asarray(det.row_of, np.int32).ravel().tolist()
     L[9] = len(L)
-    L += list(rows.ravel())
+    L += rows.ravel().tolist()
     left = getattr(det, "credit_left", None)
     if left is not None and np.any(left):
         L[16] = len(L)

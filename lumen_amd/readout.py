@@ -21,7 +21,7 @@ def pe(light, params: Params, det=None, group: int = 0):
     """Return expected photoelectrons (S,) (or (E, S) for a batched Light) at ``params``: the sensor group's keys
     are those of ``light``'s own group when it is a group's view (``light.group(name)``, the reference's
     ``readout.pe(light.group(name), params)``), else of ``det.groups[group]``."""  # noqa: D205, D209
-    import torch
+    from .api import to_device
 
     charge = light.charge
     dev, dt = charge.device, charge.dtype
@@ -37,10 +37,11 @@ def pe(light, params: Params, det=None, group: int = 0):
         eff_key = next((k for k in params.keys() if k.startswith("sensors/") and k.endswith("/efficiency")), None)
     if ce_key is None and kt > 1:
         ce_key = next((k for k in params.keys() if k.startswith("sensors/") and k.endswith("/ce")), None)
-    eff = torch.as_tensor(np.asarray(params[eff_key], np.float64), device=dev, dtype=dt) if eff_key else 1.0
+    up = lambda v: to_device(np.asarray(v, np.float64), dev).to(dt)  # noqa: E731
+    eff = up(params[eff_key]) if eff_key else 1.0
     cells = charge.reshape(*charge.shape[:-1], kl, kt)
     if kt > 1 and ce_key is not None:  # CE(theta) on its knots
-        ce = torch.as_tensor(np.asarray(params[ce_key].value, np.float64), device=dev, dtype=dt)
+        ce = up(params[ce_key].value)
         cells = (cells * ce).sum(-1)
     else:
         cells = cells.sum(-1)
@@ -48,10 +49,8 @@ def pe(light, params: Params, det=None, group: int = 0):
         return eff * cells.sum(-1)
     q = params[qe_key]
     if isinstance(q, Table):
-        qe = torch.as_tensor(np.asarray(q.value, np.float64), device=dev, dtype=dt)
-        return eff * (cells * qe).sum(-1)
-    qe = torch.as_tensor(np.asarray(q, np.float64), device=dev, dtype=dt)
-    return eff * qe * cells[..., 0]
+        return eff * (cells * up(q.value)).sum(-1)
+    return eff * up(q) * cells[..., 0]
 
 
 def pe_error(light, params: Params, det=None, group: int = 0):
