@@ -1373,7 +1373,12 @@ __global__ void __launch_bounds__(adj_block_of<F>())
 
 // the adjoint from a tape (tape.h): every photon's records read twice, in the walk's order, the same terms as the
 // replay adds from the same operands.  A lane takes the next photon of its wavefront's range that has a deposit.
-constexpr int TAPE_BLOCK = 256;
+//
+// Bound by its gathers: a load whose lanes read 64 places costs the CU some 40 cycles, and a photon's tables (its
+// medium's words, two table searches, the row's columns) are 30 of its 45 loads.  STAGED: the values, their slots and the
+// layout sit in the block's LDS, as in the photon loop (256 sources, 5.4e7 photons: 6.1 -> 4.0 ms; VALU busy 0.30
+// from memory); where four blocks a CU have no room for them they are read from memory.
+constexpr int TAPE_BLOCK = 512;
 
 // a photon's records in order
 struct TapeReader {
@@ -1404,7 +1409,7 @@ __device__ __forceinline__ void tape_leave(const Tape &T, const unsigned *left, 
   if (lane < n) T.replay[1 + at + lane] = left[lane];
 }
 
-template <unsigned F>
+template <unsigned F, bool STAGED>
 __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArgs b) {
   constexpr bool CHAN = F & F_CHAN;
   const Tape &T = a.tape;
@@ -1413,6 +1418,18 @@ __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArg
   int n_left = 0;
   double *sg = lds_cells;
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
+  if constexpr (STAGED) {
+    float *v = reinterpret_cast<float *>(sg + b.n_grad);
+    int *slot = reinterpret_cast<int *>(v + a.lds_values), *l = slot + a.lds_values;
+    for (int i = threadIdx.x; i < a.lds_values; i += blockDim.x) {
+      v[i] = a.P[i];
+      slot[i] = b.slots[i];
+    }
+    for (int i = threadIdx.x; i < a.lds_layout; i += blockDim.x) l[i] = a.L[i];
+    a.P = v;
+    b.slots = slot;
+    a.L = l;
+  }
   __syncthreads();
   const int C = a.at.classes;
   const int *row_of = a.L + a.at.row_of;
@@ -2292,7 +2309,7 @@ static int fill_args(lh_model m, Args &a, const float *values, const float *ref,
 
 // The tape of a launch of `total` photons (tape.h): the bytes it takes, 0 where the launch has none.  Measured, the
 // forward + adjoint: the tank's 2^23 photons 8.19 ms with every photon replayed, 6.64 from the tape (the walk that
-// writes it takes as long as the forward; its reader 0.9 of 6.1 ns a photon); 256 sources, 5.4e7 photons, 46.0 -> 37.6;
+// writes it takes as long as the forward; its reader 4.0 of 35 ms for 256 sources of 5.4e7 photons, which took 46.0);
 // the argon box, 2^18 photons, 435 -> 189 (the forward writes it: one walk of the longest path, not three).  It holds
 // the paths of a plain run, or of one with a WLS channel: reference values, Mie lobes, the diffusion jump, deposits at the
 // emission, acceptance angles, time histograms, torus roots and the reach bound leave it to the replay.  Up to 2^26
@@ -2519,8 +2536,7 @@ static void launch_trace(lh_model m, Args &a, int n_events, const lh_controls *c
 }
 
 // the adjoint with a tape: where the model has facet paths the walk that writes it (no tallies), then the tape's reader
-// and the replay of the photons it lists.  The reader: blocks of 256 with the gradient slots in LDS; up to 8 a CU, a
-// wavefront per 64 photons at least
+// and the replay of the photons it lists.  The reader: up to 4 blocks a CU, a wavefront per 64 photons at least
 static void launch_adjoint_tape(lh_model m, Args &a, const AdjArgs &b, const lh_controls *ctl, const Tape &t,
                                 hipStream_t st) {
   Args r = a;
@@ -2530,13 +2546,22 @@ static void launch_adjoint_tape(lh_model m, Args &a, const AdjArgs &b, const lh_
     launch_trace(m, w, 0, ctl, st, F_PATH);
   }
   const long long want = (a.total + TAPE_BLOCK - 1) / TAPE_BLOCK;
-  const int grid = (int)std::max<long long>(1, std::min<long long>(want, (long long)m->cus * 8));
+  const int grid = (int)std::max<long long>(1, std::min<long long>(want, (long long)m->cus * 4));
+  r.lds_values = (int)m->values_needed;
+  r.lds_layout = m->layout_words;
   const size_t cells = (size_t)b.n_grad * sizeof(double);
+  const size_t tables = 8 * (size_t)m->values_needed + 4 * (size_t)m->layout_words;
+  const bool staged = cells + tables + 8192 <= (size_t)m->lds_per_cu / 4;  // beside the kernel's own lists
+  const size_t bytes = cells + (staged ? tables : 0);
   hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue, t.replay);
-  if (m->has_chan)
-    hipLaunchKernelGGL(tape_adjoint_kernel<F_CHAN>, dim3(grid), dim3(TAPE_BLOCK), cells, st, r, b);
+  if (m->has_chan && staged)
+    hipLaunchKernelGGL((tape_adjoint_kernel<F_CHAN, true>), dim3(grid), dim3(TAPE_BLOCK), bytes, st, r, b);
+  else if (m->has_chan)
+    hipLaunchKernelGGL((tape_adjoint_kernel<F_CHAN, false>), dim3(grid), dim3(TAPE_BLOCK), bytes, st, r, b);
+  else if (staged)
+    hipLaunchKernelGGL((tape_adjoint_kernel<0u, true>), dim3(grid), dim3(TAPE_BLOCK), bytes, st, r, b);
   else
-    hipLaunchKernelGGL(tape_adjoint_kernel<0u>, dim3(grid), dim3(TAPE_BLOCK), cells, st, r, b);
+    hipLaunchKernelGGL((tape_adjoint_kernel<0u, false>), dim3(grid), dim3(TAPE_BLOCK), bytes, st, r, b);
   a.replay = t.replay;
   launch_adjoint(m, a, b, ctl, adjoint_lds(m, a, b, ctl), st);
 }
