@@ -210,8 +210,8 @@ int lh_adjoint(lh_model model, const float *values_dev, const float *ref_values_
  * the tape where *by_adjoint is 0; lh_adjoint_tape is lh_adjoint with the paths read from it, after writing it with one
  * walk of its own where *by_adjoint is 1 (a surface row can draw a facet path; `tape_dev` is then scratch of this call,
  * and the trace is lh_trace).  lh_tape_size gives the bytes for a launch of `photons` photons, 0 where it takes no tape
- * (reference values, more than 2^26 photons, a time grid, Mie lobes, CE knots, torus leaves, deposits at the emission,
- * `jump`, `reach_bound`): use lh_trace and lh_adjoint there.  The tape is the caller's, 16-byte aligned, and holds one
+ * (reference values, more than 2^26 photons, with a WLS channel 2^20, a time grid, Mie lobes, CE knots, torus leaves,
+ * deposits at the emission, `jump`, `reach_bound`): use lh_trace and lh_adjoint there.  The tape is the caller's, 16-byte aligned, and holds one
  * launch: values, sources, seed and controls of the adjoint are the trace's.  Photons that it has no room for are
  * replayed.  `health_dev` of the adjoint counts every photon once; its other cells are those of the replays.  No
  * counterpart in the reference. */

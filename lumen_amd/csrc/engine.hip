@@ -2308,22 +2308,25 @@ static int fill_args(lh_model m, Args &a, const float *values, const float *ref,
 }
 
 // The tape of a launch of `total` photons (tape.h): the bytes it takes, 0 where the launch has none.  Measured, the
-// forward + adjoint: the tank's 2^23 photons 8.19 ms with every photon replayed, 6.64 from the tape (the walk that
+// forward + adjoint: the tank's 2^23 photons 8.19 ms with every photon replayed, 5.90 from the tape (the walk that
 // writes it takes as long as the forward; its reader 4.0 of 35 ms for 256 sources of 5.4e7 photons, which took 46.0);
 // the argon box, 2^18 photons, 435 -> 189 (the forward writes it: one walk of the longest path, not three).  It holds
 // the paths of a plain run, or of one with a WLS channel: reference values, Mie lobes, the diffusion jump, deposits at the
 // emission, acceptance angles, time histograms, torus roots and the reach bound leave it to the replay.  Up to 2^26
-// photons: their first chunks are 4 GiB.  The pool is 64 bytes a photon beside the wavefronts' hands (the tank's mean
-// is 15), and where a channel can shift light into a slab it is caught in, 8 KiB, up to 2 GiB (the argon box takes 4.3)
-constexpr long long TAPE_MAX_PHOTONS = 1LL << 26;
+// photons: their first chunks are 4 GiB.  The pool is 512 bytes a photon, up to 2 GiB, beside the wavefronts' hands (two
+// chunks: the tank's mean is a twentieth of one), and where a channel can shift light into a slab it is caught in, 8 KiB
+// (the argon box takes 4.3), up to 8 GiB: photons past a pool's end are replayed, so a larger launch there would write
+// a tape for nothing (2^25 photons of the box with a pool for 2^18: forward 828 -> 909 ms, and the replay whole)
+constexpr long long TAPE_MAX_PHOTONS = 1LL << 26, TAPE_MAX_CAUGHT = 1LL << 20;
 
 static long long tape_bytes(lh_model m, const lh_controls *ctl, bool has_ref, long long total) {
   const bool reach = m->g.n_rnode >= 0 && ctl && ctl->reach_bound;
   if (has_ref || m->has_mie || m->NT > 0 || m->has_torus || reach || m->born_at || m->Kt > 1 || (ctl && ctl->jump) ||
-      m->layout_host[L_CLASSES] > TAPE_MAX_CLASSES || m->S > TAPE_MAX_SENSORS || total < 1 || total > TAPE_MAX_PHOTONS)
+      m->layout_host[L_CLASSES] > TAPE_MAX_CLASSES || m->S > TAPE_MAX_SENSORS || total < 1 ||
+      total > (m->has_chan ? TAPE_MAX_CAUGHT : TAPE_MAX_PHOTONS))
     return 0;
   const long long hands = 16LL * m->cus * TAPE_GRAB * 256;
-  const long long more = m->has_chan ? std::min(total * 8192, 2LL << 30) : total * 64;
+  const long long more = m->has_chan ? total * 8192 : std::min(total * 512, 2LL << 30);
   return 16 * (long long)TAPE_CONTROL + total * 64 + (hands + more) / 256 * 256 + (total + 4) / 4 * 16;
 }
 

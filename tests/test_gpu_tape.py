@@ -84,3 +84,5 @@ def test_where_a_launch_takes_no_tape(gpu):
         assert eng.tape(ctl, False, (1 << 26) + 1, by_adjoint) is None
         assert eng.tape(Controls(jump=True).struct(), False, 1000, by_adjoint) is None
     assert eng.tape(ctl, False, 1000, False) is None and eng.tape(ctl, False, 1000, True) is not None
+    argon = engine(lar_box(), "cuda")
+    assert argon.tape(ctl, False, 1000, False) is not None and argon.tape(ctl, False, (1 << 20) + 1, False) is None
