@@ -7,9 +7,9 @@
 // deposit q_k = w0 prod_{j<k} f_j g_k has the derivative q_k (sum_{j<k} dlog f_j + dlog g_k): f_j the event factor of
 // step j (attenuation, scattering density, the drawn outcome's share p_live / q), g_k the deposit's own factors
 // (reach, attenuation, the detected share).  With a cotangent c per tally cell, dL/dtheta = sum_k D_k dlog g_k +
-// sum_j dlog f_j R_{j+1}, D_k = c q_k and R_{j+1} = sum_{k>j} D_k the deposits still ahead: from a tape of its path (tape.h), or the adjoint replays each
-// photon from its Philox counter (no stored path) -- once to total T = sum_k D_k, once to add the terms with
-// R_{j+1} = T - sum_{k<=j} D_k.
+// sum_j dlog f_j R_{j+1}, D_k = c q_k and R_{j+1} = sum_{k>j} D_k the deposits still ahead: from a tape of its path
+// (tape.h), or the adjoint replays each photon from its Philox counter (no stored path) -- once to total
+// T = sum_k D_k, once to add the terms with R_{j+1} = T - sum_{k<=j} D_k.
 //
 // Pathwise terms (src/lumen/transport/step.py:318-359, :397-436): reach exp(-mu d) and attenuation exp(-mu_abs d)
 // give -d dmu, -d dmu_abs; a bulk event's density mu exp(-mu s) gives dmu / mu - s dmu.  Score terms: the surface
