@@ -256,7 +256,9 @@ class Engine:
             raise _lib.EngineError(f"the engine's tally layout ({self.stride} cells per event) is not the detector's")
         weakref.finalize(self, _lib.lib().lh_model_destroy, h)
         self.jump_grids = None  # the diffusion jump's clearance grids, built on first use
-        self._uploads = {}  # packed values by size: (the host array, its device copy), the last of each size
+        # packed values by size, the last of each: (the host array, its device copy, the stream that made it, an event
+        # after it)
+        self._uploads = {}
 
     def ensure_jump(self):
         """Build and upload the diffusion jump's clearance grids (once per engine); return them."""
@@ -345,12 +347,23 @@ class Engine:
             return None
 
     def upload(self, values: np.ndarray):
-        """Return the packed values on the device, the previous upload again when they are the same."""
+        """Return the packed values on the device, the previous upload again when they are the same.  The host does not
+        wait for the copy, so another stream than the one that made it does, and the values are kept from reuse while
+        that stream may read them."""  # noqa: D205, D209
+        import torch
+
+        current = torch.cuda.current_stream(self.device)
         last = self._uploads.get(values.nbytes)
         if last is not None and np.array_equal(last[0], values):
-            return last[1]
+            _, t, stream, copied = last
+            if stream != current:
+                current.wait_event(copied)
+                t.record_stream(current)
+            return t
         t = to_device(values, self.device)
-        self._uploads[values.nbytes] = (values.copy(), t)
+        copied = torch.cuda.Event()
+        copied.record(current)
+        self._uploads[values.nbytes] = (values.copy(), t, current, copied)
         return t
 
 
