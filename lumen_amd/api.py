@@ -224,11 +224,16 @@ def moment_error(q2, s, n: int):
 def to_device(a: np.ndarray, device):
     """Return the array on the device, copied on the current stream without waiting for it: a copy from pageable memory
     waits for all the stream holds, the photon loop launched before it included (a call of 10^5 photons in the tank
-    then takes its host time and its kernel's one after the other)."""  # noqa: D205, D209
+    then takes its host time and its kernel's one after the other).  Refused while a graph is captured: a replay would
+    copy whatever the pinned memory holds by then."""  # noqa: D205, D209
     import torch
 
     t = torch.from_numpy(np.array(a))
-    return t.pin_memory().to(device, non_blocking=True) if torch.device(device).type == "cuda" else t.to(device)
+    if torch.device(device).type != "cuda":
+        return t.to(device)
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a host array cannot be uploaded while a graph is captured: upload it before the capture")
+    return t.pin_memory().to(device, non_blocking=True)
 
 
 class Engine:
