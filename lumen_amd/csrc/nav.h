@@ -713,9 +713,10 @@ __device__ inline Cross query_t(const Geo &g, float3 x, float3 d, int vol, int l
     int v2 = best.vol_after;
     if (best.own) {
       const int near = g.vinfo[vol].x;
+      const bool deep = (near & 2) && best.t > 0.0f;  // an exit at 0: the start may lie outside vol, anywhere (lh_query)
       float3 xl, dl;
-      if (!(near & 2)) to_local(g, best.vol_after, xp, d, xl, dl);
-      if (!(near & 2) && !solid_inside<TOR>(g, g.vkind[best.vol_after], xl)) v2 = locate<TOR>(g, xp);
+      if (!deep) to_local(g, best.vol_after, xp, d, xl, dl);
+      if (!deep && !solid_inside<TOR>(g, g.vkind[best.vol_after], xl)) v2 = locate<TOR>(g, xp);
       else if (near & 1) v2 = locate<TOR>(g, xp, best.vol_after);
     } else {
       const int2 gr = g.vgrp[best.vol_after];
