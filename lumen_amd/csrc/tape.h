@@ -81,13 +81,18 @@ __device__ inline void tape_put(const Tape &T, TapePos &t, uint4 r) {
     volatile unsigned *hand = s_pool[threadIdx.x >> 6];  // one cell for these lanes: the branches on it are uniform
     unsigned base = hand[0];
     if (base + cnt > hand[1]) {
-      unsigned got = 0;
-      if (rank == 0) got = atomicAdd(&T.cells[0].x, (unsigned)TAPE_GRAB);
-      base = (unsigned)__builtin_amdgcn_readfirstlane((int)got);
-      const bool out = base + TAPE_GRAB > T.pool || base + TAPE_GRAB < base;
-      if (rank == 0) {
-        hand[0] = base;
-        hand[1] = out ? base : base + TAPE_GRAB;
+      // a wavefront whose hand begins in the pool's last chunks would get a later one: it asks no more, so the pool's
+      // counter ends at most one grab a wavefront past the pool
+      bool out = base + TAPE_GRAB > T.pool;
+      if (!out) {
+        unsigned got = 0;
+        if (rank == 0) got = atomicAdd(&T.cells[0].x, (unsigned)TAPE_GRAB);
+        base = (unsigned)__builtin_amdgcn_readfirstlane((int)got);
+        out = base + TAPE_GRAB > T.pool;
+        if (rank == 0) {
+          hand[0] = base;
+          hand[1] = out ? base : base + TAPE_GRAB;
+        }
       }
       if (out) {
         t.n = -1;

@@ -1,0 +1,38 @@
+"""A tape whose pool runs out: the pool's counter stops, and the photons left without are replayed."""
+
+import numpy as np
+import pytest
+
+from test_gpu_tape import _both, _run
+from toys import sphere_toy
+
+pytestmark = pytest.mark.gpu
+
+KEY = ("surfaces/Wall/REFLECTIVITY",)
+
+
+def _sphere(facets, n):
+    """A bright sphere of some 460 vertices a photon (with facets half of its reflections are facet paths)."""
+    extra = dict(p_spike=0.0, p_lobe=0.5, p_back=0.0, sigma_alpha=0.2)
+    det = sphere_toy(1.0, "UNIFIED_METAL" if facets else "PAINTED", R=0.99, L_abs=1e3, extra=extra if facets else None)
+    return _run(det, KEY, (0.1, 0.0, 0.0), 400.0, (n,))
+
+
+def _pool(tape, n):
+    """The pool's chunks: the tape less its control cells, first chunks and replay list."""
+    return (tape.numel() // 16 - 4 - 4 * n - (n + 4) // 4) // 16
+
+
+@pytest.mark.parametrize("facets", [False, True])
+def test_the_pools_counter_stops(gpu, facets):
+    """Each wavefront asks an empty pool once: a counter that grew with every photon would wrap at 2^26 of them, and
+    chunks would be handed out twice."""
+    import torch
+
+    n = 100_000
+    run = _sphere(facets, n)
+    a, b, tape = _both(run)
+    asked, pool = int(tape[:4].view(torch.int32).item()), _pool(tape, n)
+    waves = 12 * run.eng.last_launch()["grid"]
+    assert pool < asked <= pool + 64 * waves
+    assert np.linalg.norm(b - a) <= 2e-6 * np.linalg.norm(a)
