@@ -1292,6 +1292,7 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
     if (alive) {
       alive = step<false, F>(a, p, acc, nullptr, nullptr);
       if constexpr ((F & F_TAPE) != 0) tape_step<(F & F_CHAN) != 0, (F & F_PATH) != 0>(a.tape, p.tape, p.rec, p.lam);
+      if constexpr ((F & F_PATH) != 0) alive = alive && p.tape.n >= 0;  // no room for its path: the replay walks it
       if (!alive) {
         if constexpr ((F & F_PATH) == 0) photon_end(a, p);
         if constexpr ((F & F_TAPE) != 0) tape_end(a.tape, p.tape, (unsigned)p.gi, p.event);

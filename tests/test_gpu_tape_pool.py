@@ -1,5 +1,7 @@
 """A tape whose pool runs out: the pool's counter stops, and the photons left without are replayed."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -36,3 +38,27 @@ def test_the_pools_counter_stops(gpu, facets):
     waves = 12 * run.eng.last_launch()["grid"]
     assert pool < asked <= pool + 64 * waves
     assert np.linalg.norm(b - a) <= 2e-6 * np.linalg.norm(a)
+
+
+def _ms(run, tape):
+    """The adjoint's time, the best of three after a first."""
+    import torch
+
+    out = []
+    for _ in range(4):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        run._launch_adjoint(tape=tape)
+        torch.cuda.synchronize()
+        out.append(1e3 * (time.perf_counter() - t0))
+    return min(out[1:])
+
+
+@pytest.mark.parametrize("n", [1 << 20])
+def test_an_empty_pool_costs_little(gpu, n):
+    """Most photons find no room: the adjoint's own walk ends them there (a walk to their end, then the two of the
+    replay, took 1.4 times the replay).  A quarter is room for the taped share's walk and the clocks."""
+    run = _sphere(True, n)
+    a, b, tape = _both(run)
+    assert np.linalg.norm(b - a) <= 2e-6 * np.linalg.norm(a)
+    assert _ms(run, tape) <= 1.25 * _ms(run, None)
