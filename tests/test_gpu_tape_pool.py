@@ -31,7 +31,7 @@ def test_the_pools_counter_stops(gpu, facets):
     chunks would be handed out twice."""
     import torch
 
-    n = 100_000
+    n = 1 << 20
     run = _sphere(facets, n)
     a, b, tape = _both(run)
     asked, pool = int(tape[:4].view(torch.int32).item()), _pool(tape, n)
