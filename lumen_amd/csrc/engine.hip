@@ -1209,6 +1209,36 @@ __device__ inline Args stage_tables(const Args &a0) {
   return a;
 }
 
+// How a launch's photons are handed out (Range).  An explicit chunk is every range's size.  Else, by the photons a
+// wavefront gets when all are handed out at once: up to STATIC_SHARE the first ranges hold them all, no queue, the
+// photons on as many wavefronts as there are (tank, 100,003 photons: 0.14 ms, 0.28 in chunks of 256 that fill an
+// eighth of the wavefronts; the tutorial's 2^18: 0.05 against 0.08); beyond it the first ranges hold three quarters
+// and the queue evens out the rest in small chunks (tank, 2^22 photons: 1.28 ms, 1.42 in chunks of 256 from the start,
+// whose last ones the launch waits for; 2^24: 4.69 against 4.77).  At the line both take the same (tank, 2^20: 0.44
+// and 0.43 ms).  Chunks of 64 to 128: below, the claims (12 ns each, one address) show on cheap photons.
+constexpr long long STATIC_SHARE = 384;
+constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
+
+// the split of the launch's photons over `waves` wavefronts (`given`: in chunks of the controls' size)
+__host__ __device__ inline void split_photons(Args &a, long long waves, bool given) {
+  long long first = a.chunk;
+  if (!given) {
+    const long long share = (a.total + waves - 1) / waves, part = share / 16;
+    first = share <= STATIC_SHARE ? share : share / 4 * 3;
+    a.chunk = (int)(part < MIN_CHUNK ? MIN_CHUNK : part > MAX_CHUNK ? MAX_CHUNK : part);
+  }
+  a.first_chunk = first;
+  a.dyn_at = a.total < waves * first ? a.total : waves * first;
+}
+
+// ... of the photons a tape left to the replay, their number known on the device alone.  The queue matters here too: with an
+// equal share for every wavefront the launch waits for the one that got the longest paths (a sphere with facets, R 0.99,
+// 2^22 photons, three quarters of them replayed: adjoint 137 ms, 110 with the queue)
+__device__ __forceinline__ void split_replay(Args &a) {
+  a.total = (long long)(unsigned)__builtin_amdgcn_readfirstlane((int)a.replay[0]);
+  split_photons(a, (long long)gridDim.x * (blockDim.x >> 6), a.chunk > 0);
+}
+
 // A wavefront's range of the launch's photons.  Its first is its own by its index, wavefront w of every block before
 // wavefront w + 1 of any (a launch of few photons spreads over the CUs), so a launch begins without a claim: the
 // atomics on one address take 12 ns each, 37 us for the 3,072 wavefronts' first claims.  Past the first ranges the
@@ -1224,17 +1254,9 @@ __device__ __forceinline__ Range first_range(const Args &a) {
   return Range{b, min(b + a.first_chunk, a.dyn_at), false};
 }
 
-// ... and of the photons a tape left to the replay: as many of the list for every wavefront
-__device__ __forceinline__ Range replay_range(const Args &a) {
-  const unsigned waves = gridDim.x * (blockDim.x >> 6), n = a.replay[0], share = (n + waves - 1) / waves;
-  const unsigned w = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-  const unsigned b = min(w * share, n);
-  return Range{(long long)b, (long long)min(b + share, n), false};
-}
-
 // the next chunk when the range is used up: false once there is none
 __device__ __forceinline__ bool next_range(const Args &a, Range &r, int lane) {
-  if (a.dyn_at < a.total && !a.replay) {
+  if (a.dyn_at < a.total) {
     unsigned long long c = 0;
     if (lane == 0) c = atomicAdd(a.queue, (unsigned long long)a.chunk);
     const long long base = a.dyn_at + (long long)__shfl(c, 0);
@@ -1324,13 +1346,14 @@ __global__ void __launch_bounds__(adj_block_of<F>())
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
   clear_block_cells();
   stage_nodes(a0.g);
-  const Args a = stage_tables<F>(a0);
+  Args a = stage_tables<F>(a0);
+  if (a.replay) split_replay(a);
   __syncthreads();
   Photon p;
   Acc acc{};
   bool alive = false;
   const int lane = threadIdx.x & 63;
-  Range r = a.replay ? replay_range(a) : first_range(a);
+  Range r = first_range(a);
   for (;;) {
     bool need = !alive;
     unsigned long long mask = __ballot(need);
@@ -2369,6 +2392,7 @@ static unsigned features_of(lh_model m, const Args &a, bool adj) {
 
 
 
+
 // the workgroup size of a launch's kernel
 static int block_for(bool /* adjoint or forward */, unsigned /* features */) { return BLOCK; }
 
@@ -2477,27 +2501,10 @@ static size_t place_lds(lh_model m, Args &a, const void *fn, int block, size_t c
   return end;
 }
 
-// How a launch's photons are handed out (Range).  An explicit chunk is every range's size.  Else, by the photons a
-// wavefront gets when all are handed out at once: up to STATIC_SHARE the first ranges hold them all, no queue, the
-// photons on as many wavefronts as there are (tank, 100,003 photons: 0.14 ms, 0.28 in chunks of 256 that fill an
-// eighth of the wavefronts; the tutorial's 2^18: 0.05 against 0.08); beyond it the first ranges hold three quarters
-// and the queue evens out the rest in small chunks (tank, 2^22 photons: 1.28 ms, 1.42 in chunks of 256 from the start,
-// whose last ones the launch waits for; 2^24: 4.69 against 4.77).  At the line both take the same (tank, 2^20: 0.44
-// and 0.43 ms).  Chunks of 64 to 128: below, the claims (12 ns each, one address) show on cheap photons.
-constexpr long long STATIC_SHARE = 384;
-constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
-
 static void claim_schedule(Args &a, const lh_controls *ctl, int grid, int block, hipStream_t st) {
-  const long long waves = (long long)grid * (block / 64);
-  long long first = a.chunk;
-  if (!(ctl && ctl->chunk > 0)) {
-    const long long share = (a.total + waves - 1) / waves;
-    first = share <= STATIC_SHARE ? share : share / 4 * 3;
-    a.chunk = (int)std::min(std::max(share / 16, MIN_CHUNK), MAX_CHUNK);
-  }
-  a.first_chunk = first;
-  a.dyn_at = std::min(a.total, waves * first);
-  if ((a.dyn_at < a.total && !a.replay) || a.tape.cells)
+  if (a.replay) return;  // split on the device, its queue cleared before the reader
+  split_photons(a, (long long)grid * (block / 64), ctl && ctl->chunk > 0);
+  if (a.dyn_at < a.total || a.tape.cells)
     hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue, a.tape.cells ? &a.tape.cells[0].x : nullptr);
 }
 

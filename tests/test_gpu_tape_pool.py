@@ -54,11 +54,28 @@ def _ms(run, tape):
     return min(out[1:])
 
 
-@pytest.mark.parametrize("n", [1 << 20])
+@pytest.mark.parametrize("n", [1 << 20, 1 << 22])
 def test_an_empty_pool_costs_little(gpu, n):
     """Most photons find no room: the adjoint's own walk ends them there (a walk to their end, then the two of the
-    replay, took 1.4 times the replay).  A quarter is room for the taped share's walk and the clocks."""
+    replay, took 1.4 times the replay), and the replay evens them out over the wavefronts (equal shares of 2^22 took
+    another 1.4).  A quarter is room for the taped share's walk and the clocks."""
     run = _sphere(True, n)
     a, b, tape = _both(run)
     assert np.linalg.norm(b - a) <= 2e-6 * np.linalg.norm(a)
     assert _ms(run, tape) <= 1.25 * _ms(run, None)
+
+
+@pytest.mark.parametrize("n,chunk", [(100_001, 100), (1 << 18, 64), (1 << 21, 0), ((1 << 21) + 63, 1 << 20)])
+def test_every_photon_left_is_replayed_once(gpu, n, chunk):
+    """The replay of a list in first ranges alone, with the work queue's chunks, and in chunks larger than the list."""
+    from lumen_amd import _lib
+    from lumen_amd.api import Controls
+
+    run = _sphere(True, n)
+    a, _, tape = _both(run)
+    run.grad.zero_()
+    run.adj_health.zero_()
+    run._launch_adjoint(Controls(chunk=chunk), tape=tape)
+    b = run.grad.cpu().numpy()
+    assert float(run.adj_health.cpu()[_lib.HEALTH_NAMES.index("photons")]) == n
+    assert np.linalg.norm(b - a) <= 2e-6 * np.linalg.norm(a)
