@@ -112,20 +112,28 @@ def _function():
 
     class PhotonLoop(torch.autograd.Function):
         """tally = photon_loop(values): forward lh_trace, backward lh_adjoint.  Where the launch takes a tape, the
-        forward of a detector without facet paths writes it (saved beside the values), else the backward itself."""
+        forward of a detector without facet paths writes it, else the backward itself.
+
+        The tape is an attribute of a saved empty tensor: it lives as long as the saved values do, and hooks on saved
+        tensors do not get it.  A tape has up to gigabytes and links that the kernel follows, so it is not to be moved,
+        packed or rounded; where a hook hands another tensor back, the photons are replayed."""
 
         @staticmethod
         def forward(ctx, values, run):
             ctx.run = run
-            tape = None
+            tape = mark = None
             if ctx.needs_input_grad[0]:
                 tape = _tape(run, False)
-            ctx.save_for_backward(values, tape)
+            if tape is not None:
+                mark = values.new_empty(0)
+                mark.tape = tape
+            ctx.save_for_backward(values, mark)
             return _trace(run, values.detach().contiguous(), tape)
 
         @staticmethod
         def backward(ctx, g):
-            values, tape = ctx.saved_tensors
+            values, mark = ctx.saved_tensors
+            tape = getattr(mark, "tape", None)
             run = ctx.run
             if tape is None:
                 tape = _tape(run, True)
