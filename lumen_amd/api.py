@@ -12,6 +12,7 @@ photons are the same however it is split (the reference's ``first_id`` chunks, `
 
 from __future__ import annotations
 
+import threading
 import weakref
 from dataclasses import dataclass, field
 from typing import Any, NamedTuple
@@ -236,6 +237,21 @@ def to_device(a: np.ndarray, device):
     return t.pin_memory().to(device, non_blocking=True)
 
 
+# The tapes alive, over all engines.  Together on a device they take at most one part in TAPE_PARTS of the memory that
+# would be free there without them, so results kept for a later backward (one tape each where the forward writes it) leave
+# the rest to the program: past that a launch takes no tape and its adjoint replays the photons, which needs no memory.
+TAPE_PARTS = 8
+_TAPES: "weakref.WeakSet[_Held]" = weakref.WeakSet()
+_TAPES_LOCK = threading.Lock()
+
+
+class _Held:
+    """One tape's bytes, alive as long as the tape's tensor, which carries it."""
+
+    def __init__(self, nbytes: int, device: int):
+        self.nbytes, self.device = nbytes, device
+
+
 class Engine:
     """A detector's model on the device (built once per detector and device) and its run state."""
 
@@ -337,8 +353,8 @@ class Engine:
 
     def tape(self, ctl, has_ref: bool, photons: int, adjoint: bool):
         """Return a tape (a uint8 device tensor) for a launch of ``photons`` photons whose adjoint follows
-        (``adjoint``: for its adjoint), or None where that launch writes none or the device has no room for it (the
-        adjoint then replays the photons)."""  # noqa: D205, D209
+        (``adjoint``: for its adjoint), or None where that launch writes none or the tapes would take more than their
+        part of the device's free memory (the adjoint then replays the photons)."""  # noqa: D205, D209
         import torch
 
         size, by_adjoint = _lib.C.c_int64(), _lib.C.c_int32()
@@ -346,10 +362,19 @@ class Engine:
                                            _lib.C.byref(size), _lib.C.byref(by_adjoint)), "lh_tape_size")
         if size.value == 0 or bool(by_adjoint.value) != adjoint:
             return None
+        device = torch.device(self.device).index
+        held = _Held(size.value, torch.cuda.current_device() if device is None else device)
+        with _TAPES_LOCK:
+            taken = sum(h.nbytes for h in _TAPES if h.device == held.device)
+            if TAPE_PARTS * (taken + held.nbytes) > taken + torch.cuda.mem_get_info(held.device)[0]:
+                return None
+            _TAPES.add(held)
         try:
-            return torch.empty(size.value, dtype=torch.uint8, device=self.device)
+            tape = torch.empty(held.nbytes, dtype=torch.uint8, device=self.device)
         except torch.cuda.OutOfMemoryError:
             return None
+        tape.held = held
+        return tape
 
     def upload(self, values: np.ndarray):
         """Return the packed values on the device, the previous upload again when they are the same.  The host does not
