@@ -46,7 +46,9 @@ def _key(run, what):
     import torch
 
     name = torch.cuda.get_device_name(run.eng.device)
-    return f"{run.det.name}|{what}|photons={run.total}|sources={len(run.rows)}|{name}"
+    # the chunks it was chosen from: a choice made among others is timed again
+    chunks = ",".join(map(str, CHUNKS if what == "forward" else ADJ_CHUNKS))
+    return f"{run.det.name}|{what}|photons={run.total}|sources={len(run.rows)}|chunks={chunks}|{name}"
 
 
 ADJ_CHUNKS = (0, 128, 512, 2048)  # the adjoint's launches cost ~4 forward ones: a coarser grid, timed once each
