@@ -61,7 +61,7 @@ class BatchRun:
             self.eng.ensure_jump()
         self._g_fwd = self._g_both = None
         self._loss = None
-        self._tape = None  # forward_adjoint's: the photons' paths, for its adjoint
+        self._tape = self._tape_of = None  # forward_adjoint's: the photons' paths, for its adjoint; the controls' paths
 
     def close(self):
         """Release the batch's device buffers (its sources and work queue); the captured graphs go with them."""
@@ -121,6 +121,20 @@ class BatchRun:
         self.adj_health.zero_()
         self._launch_adjoint(tape=self._tape)
 
+    def _choose_tape(self):
+        """Set the tape of this run's forward and adjoint (None: it takes none), anew where its controls were replaced
+        since.  A tape holds the forward's paths: the adjoint's controls are to ask for the same ones."""  # noqa: D205, D209
+        shape = dict(chunk=0, blocks_per_cu=0, tally_global=False, nodes_global=False)
+        paths = tuple(c._replace(**shape) for c in (self.controls, self.adj_controls or Controls()))
+        if self._tape_of == paths:
+            return
+        self._tape_of, self._tape, self._g_both = paths, None, None  # a captured graph holds the tape's address
+        if paths[0] == paths[1]:
+            ctl = self.controls.struct()
+            self._tape = self.eng.tape(ctl, False, self.total, False)
+            if self._tape is None:
+                self._tape = self.eng.tape(ctl, False, self.total, True)
+
     def _capture(self, body):
         import torch
 
@@ -151,11 +165,8 @@ class BatchRun:
         slots (n_grad,).  Captured as one graph on first use (the loss function is part of it)."""  # noqa: D205, D209
         if self._loss is not loss:
             self._loss, self._g_both = loss, None
-        if self._tape is None and self._g_both is None and self.has_grad:
-            ctl = self.controls.struct()
-            self._tape = self.eng.tape(ctl, False, self.total, False)
-            if self._tape is None:
-                self._tape = self.eng.tape(ctl, False, self.total, True)
+        if self.has_grad and (self._g_both is None or not self.graph):
+            self._choose_tape()
         if self.adj_controls is None and self._tape is not None:
             self.adj_controls = Controls()  # the adjoint reads the tape: no walk whose launch shape matters
         if self.adj_controls is None:  # the adjoint's launch shape: tuned once, with this loss's cotangent
