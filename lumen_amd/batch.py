@@ -168,7 +168,9 @@ class BatchRun:
         if self.has_grad and (self._g_both is None or not self.graph):
             self._choose_tape()
         if self.adj_controls is None and self._tape is not None:
-            self.adj_controls = Controls()  # the adjoint reads the tape: no walk whose launch shape matters
+            # the adjoint's walks are the forward's (the one that writes the tape, where a surface can draw facets) or
+            # the replay of what the tape had no room for: the forward's launch shape
+            self.adj_controls = self.controls
         if self.adj_controls is None:  # the adjoint's launch shape: tuned once, with this loss's cotangent
             self._fwd_body()
             self.cot.copy_(loss(self.tally))

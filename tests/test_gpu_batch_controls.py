@@ -72,3 +72,17 @@ def test_an_eager_call_between_replays(gpu):
     for _ in range(2):
         b = run.forward_adjoint(loss).cpu().numpy()
         assert np.linalg.norm(b - a) <= 2e-6 * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("where", sorted(DETS))
+def test_the_adjoint_of_a_tape_has_the_forwards_launch_shape(gpu, where, monkeypatch):
+    from lumen_amd import batch
+
+    monkeypatch.setattr(batch, "tuned_controls", lambda run, what: Controls(chunk=192))
+    mk, keys, lam, n = DETS[where]
+    src = Batch((Point((0.3, 0.2, -0.1), lam=lam, n_photons=float(n)),), (n,))
+    tuned = BatchRun(mk(), src, seed=3, grad_keys=keys, graph=False)
+    plain = BatchRun(mk(), src, seed=3, grad_keys=keys, graph=False, tune=False)
+    a, b = (r.forward_adjoint(_loss(r)).cpu().numpy() for r in (tuned, plain))
+    assert tuned._tape is not None and tuned.adj_controls.chunk == tuned.controls.chunk == 192
+    assert np.linalg.norm(a - b) <= 2e-6 * np.linalg.norm(b)
