@@ -67,7 +67,8 @@ def test_an_empty_pool_costs_little(gpu, n):
 
 @pytest.mark.parametrize("n,chunk", [(100_001, 100), (1 << 18, 64), (1 << 21, 0), ((1 << 18) + 63, 2048)])
 def test_every_photon_left_is_replayed_once(gpu, n, chunk):
-    """The replay of a list in first ranges alone, with the work queue's chunks, and in chunks that a few wavefronts take all of."""
+    """The replay of a list in first ranges alone, with the work queue's chunks, and in chunks that a few wavefronts
+    take all of."""
     from lumen_amd import _lib
     from lumen_amd.api import Controls
 
