@@ -9,7 +9,7 @@
 // the photon's summed deposits to `arrival2` (the per-photon second moment).
 //
 // Schedule: each wavefront keeps 64 photons in flight; a lane whose photon ended takes the next one from its
-// wavefront's range, a first one of its own and then chunks claimed from the device work queue (one atomic per chunk),
+// wavefront's range, blocks of its own first and then chunks claimed from the device work queue (one atomic per chunk),
 // so lanes refill every step (the reference's
 // "step" schedule, src/lumen/run.py:81) and a launch of many sources with uneven photon counts keeps every lane busy.
 #include <hip/hip_runtime.h>
@@ -99,8 +99,9 @@ struct Args {
   uint32_t k0, k1;
   float roulette, max_dist, reach;
   int max_vert, chunk;
-  long long first_chunk;  // the photons of each wavefront's first range, its own by its index (claim_schedule)
-  long long dyn_at;       // where the first ranges end: the work queue hands out the photons past it, chunk by chunk
+  long long block, stride;  // each wavefront's own blocks of photons: their size, the step from one to its next (Range)
+  long long dyn_at, rows;   // where the own blocks end: the work queue hands out the photons past it, in QUEUE_PARTS
+                            // parts of `rows` chunks each
   int keep_zero;  // 1: a photon whose live weight became 0 walks on (the reference's records); 0: it ends
   int reach_on;   // 1: the reach bound where the model has one (the controls' reach_bound)
   double *__restrict__ tally;
@@ -1209,26 +1210,36 @@ __device__ inline Args stage_tables(const Args &a0) {
   return a;
 }
 
-// How a launch's photons are handed out (Range).  An explicit chunk is every range's size.  Else, by the photons a
-// wavefront gets when all are handed out at once: up to STATIC_SHARE the first ranges hold them all, no queue, the
-// photons on as many wavefronts as there are (tank, 100,003 photons: 0.14 ms, 0.28 in chunks of 256 that fill an
-// eighth of the wavefronts; the tutorial's 2^18: 0.05 against 0.08); beyond it the first ranges hold three quarters
-// and the queue evens out the rest in small chunks (tank, 2^22 photons: 1.28 ms, 1.42 in chunks of 256 from the start,
-// whose last ones the launch waits for; 2^24: 4.69 against 4.77).  At the line both take the same (tank, 2^20: 0.44
-// and 0.43 ms).  Chunks of 64 to 128: below, the claims (12 ns each, one address) show on cheap photons.
-constexpr long long STATIC_SHARE = 384;
+// How a launch's photons are handed out (Range).  An explicit chunk is every block's size.  Else each wavefront has up to
+// OWN_PHOTONS of its own, in blocks of at most 64, and the work queue hands out the rest in small chunks.  Measured in the
+// tank, the kernel: 2^17 photons, all of them own, 0.14 ms, 0.28 in chunks of 256 that fill a sixth of the wavefronts;
+// 2^20 0.43 against 0.48; 2^22 1.26 against 1.36; 2^24 4.63 against 4.65.  Chunks of 64 to 128: below, the claims (12 ns
+// each, one address) show on cheap photons.
+// Paths differ from source to source, so no wavefront may be left with many photons of one: its own blocks lie a stride of
+// all wavefronts apart, and 256 photons are what a queue of usual chunks would give it at once.  64 sources of which
+// every eighth has long paths (a sphere, 270 vertices against 1), 2^22 photons: 9.7 ms, 39.6 with three quarters of the
+// launch in equal shares of consecutive photons, 13.7 in chunks of 256.  The queue deals its chunks out of QUEUE_PARTS
+// parts of the launch in turn: taken in order, every wavefront would be at one source's photons at a time, and where the
+// events' tallies are in memory at one event's cells (256 sources in the tank, 5.4e7 photons: 16.8 ms in order, 15.5 so).
+constexpr long long OWN_PHOTONS = 256;
 constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
+constexpr int QUEUE_PARTS_LOG = 6, QUEUE_PARTS = 1 << QUEUE_PARTS_LOG;
 
 // the split of the launch's photons over `waves` wavefronts (`given`: in chunks of the controls' size)
 __host__ __device__ inline void split_photons(Args &a, long long waves, bool given) {
-  long long first = a.chunk;
+  long long count = 1;  // own blocks
+  a.block = a.chunk;
   if (!given) {
-    const long long share = (a.total + waves - 1) / waves, part = share / 16;
-    first = share <= STATIC_SHARE ? share : share / 4 * 3;
-    a.chunk = (int)(part < MIN_CHUNK ? MIN_CHUNK : part > MAX_CHUNK ? MAX_CHUNK : part);
+    const long long share = (a.total + waves - 1) / waves, some = share / 16;
+    const long long own = share < OWN_PHOTONS ? share : OWN_PHOTONS;
+    a.chunk = (int)(some < MIN_CHUNK ? MIN_CHUNK : some > MAX_CHUNK ? MAX_CHUNK : some);
+    count = (own + MIN_CHUNK - 1) / MIN_CHUNK;
+    a.block = own > 0 ? (own + count - 1) / count : 0;
   }
-  a.first_chunk = first;
-  a.dyn_at = a.total < waves * first ? a.total : waves * first;
+  a.stride = waves * a.block;
+  a.dyn_at = a.total < a.stride * count ? a.total : a.stride * count;
+  const long long row = (long long)QUEUE_PARTS * a.chunk;
+  a.rows = (a.total - a.dyn_at + row - 1) / row;
 }
 
 // ... of the photons a tape left to the replay, their number known on the device alone.  The queue matters here too: with an
@@ -1239,10 +1250,10 @@ __device__ __forceinline__ void split_replay(Args &a) {
   split_photons(a, (long long)gridDim.x * (blockDim.x >> 6), a.chunk > 0);
 }
 
-// A wavefront's range of the launch's photons.  Its first is its own by its index, wavefront w of every block before
-// wavefront w + 1 of any (a launch of few photons spreads over the CUs), so a launch begins without a claim: the
-// atomics on one address take 12 ns each, 37 us for the 3,072 wavefronts' first claims.  Past the first ranges the
-// wavefront claims chunks from the work queue; a launch whose first ranges hold every photon never touches it.
+// A wavefront's range of the launch's photons.  Its first blocks are its own by its index, wavefront w of every workgroup
+// before wavefront w + 1 of any (a launch of few photons spreads over the CUs), so a launch begins without a claim: the
+// atomics on one address take 12 ns each, 37 us for the 3,072 wavefronts' first claims.  Past them the wavefront claims
+// chunks from the work queue, by their number; a launch whose own blocks hold every photon never touches it.
 struct Range {
   long long cursor, end;
   bool drained;
@@ -1250,16 +1261,28 @@ struct Range {
 
 __device__ __forceinline__ Range first_range(const Args &a) {
   const long long w = (long long)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-  const long long b = min(w * a.first_chunk, a.dyn_at);
-  return Range{b, min(b + a.first_chunk, a.dyn_at), false};
+  const long long b = w * a.block;
+  return Range{min(b, a.dyn_at), min(b + a.block, a.dyn_at), false};
 }
 
-// the next chunk when the range is used up: false once there is none
+// the next block or chunk when the range is used up: false once there is none.  The next own block lies a stride past the
+// one that ends; only the launch's last is cut short, at dyn_at.  The parts are equal but for the last, which may hold fewer
+// chunks than it has numbers
 __device__ __forceinline__ bool next_range(const Args &a, Range &r, int lane) {
-  if (a.dyn_at < a.total) {
+  const long long next = r.end - a.block + a.stride;
+  if (r.end < a.dyn_at && next < a.dyn_at) {
+    r.cursor = next;
+    r.end = min(next + a.block, a.dyn_at);
+    return true;
+  }
+  while (a.dyn_at < a.total) {
     unsigned long long c = 0;
-    if (lane == 0) c = atomicAdd(a.queue, (unsigned long long)a.chunk);
-    const long long base = a.dyn_at + (long long)__shfl(c, 0);
+    if (lane == 0) c = atomicAdd(a.queue, 1ull);
+    c = __shfl(c, 0);
+    const long long row = (long long)(c >> QUEUE_PARTS_LOG);
+    if (row >= a.rows) break;
+    const long long part = (long long)(c & (QUEUE_PARTS - 1));
+    const long long base = a.dyn_at + (part * a.rows + row) * a.chunk;
     if (base < a.total) {
       r.cursor = base;
       r.end = min(base + a.chunk, a.total);
@@ -1288,7 +1311,8 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
   Range r = first_range(a);
   for (;;) {
     // refill the lanes whose photon ended from the wavefront's chunk of the work queue
-    bool need = !alive;
+    bool need = !alive, taken = false;
+    long long gi = 0;
     unsigned long long mask = __ballot(need);
     while (mask != 0ull && !r.drained) {
       const long long avail = r.end - r.cursor;
@@ -1299,16 +1323,20 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
       const int rank = lanes_below(mask);
       const bool take = need && rank < avail;
       if (take) {
-        alive = emit<(F & F_TORUS) != 0>(a, r.cursor + rank, p, acc);
-        if constexpr ((F & F_TAPE) != 0) {
-          p.gi = r.cursor + rank;
-          tape_begin(p.tape, (unsigned)p.gi, p.lam);
-          if (!alive) tape_end(a.tape, p.tape, (unsigned)p.gi, p.event);
-        }
+        gi = r.cursor + rank;
+        taken = true;
       }
       r.cursor += min((long long)__popcll(mask), avail);
       need = need && !take;
       mask = __ballot(need);
+    }
+    if (taken) {  // once, where a range ended in the middle too
+      alive = emit<(F & F_TORUS) != 0>(a, gi, p, acc);
+      if constexpr ((F & F_TAPE) != 0) {
+        p.gi = gi;
+        tape_begin(p.tape, (unsigned)p.gi, p.lam);
+        if (!alive) tape_end(a.tape, p.tape, (unsigned)p.gi, p.event);
+      }
     }
     if (!__any(alive) && r.drained) break;
     if (alive) {
@@ -1355,7 +1383,8 @@ __global__ void __launch_bounds__(adj_block_of<F>())
   const int lane = threadIdx.x & 63;
   Range r = first_range(a);
   for (;;) {
-    bool need = !alive;
+    bool need = !alive, taken = false;
+    long long gi = 0;
     unsigned long long mask = __ballot(need);
     while (mask != 0ull && !r.drained) {
       const long long avail = r.end - r.cursor;
@@ -1366,15 +1395,19 @@ __global__ void __launch_bounds__(adj_block_of<F>())
       const int rank = lanes_below(mask);
       const bool take = need && rank < avail;
       if (take) {
-        p.gi = a.replay ? (long long)a.replay[1 + r.cursor + rank] : r.cursor + rank;
-        alive = emit<(F & F_TORUS) != 0>(a, p.gi, p, acc);
-        p.pass = 0;
-        p.T = p.Dsum = 0.0f;
-        p.hasdep = false;
+        gi = r.cursor + rank;
+        taken = true;
       }
       r.cursor += min((long long)__popcll(mask), avail);
       need = need && !take;
       mask = __ballot(need);
+    }
+    if (taken) {
+      p.gi = a.replay ? (long long)a.replay[1 + gi] : gi;
+      alive = emit<(F & F_TORUS) != 0>(a, p.gi, p, acc);
+      p.pass = 0;
+      p.T = p.Dsum = 0.0f;
+      p.hasdep = false;
     }
     if (!__any(alive) && r.drained) break;
     if (alive) {
@@ -1459,9 +1492,10 @@ __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArg
   const int *row_of = a.L + a.at.row_of;
   const unsigned waves = gridDim.x * (TAPE_BLOCK / 64);
   const unsigned w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-  const unsigned share = (T.photons + waves - 1) / waves;
-  unsigned cursor = min(w * share, T.photons);
-  const unsigned end = min(cursor + share, T.photons);
+  // 64 photons at a time, a stride of all wavefronts apart: the photons with long paths, or with a tape at all where the
+  // pool ran out, lie side by side (a sphere with facets, 2^22 photons, the first third of them on tape: 24.6 ms in equal
+  // shares of consecutive photons, 9.9 so)
+  unsigned block = w * 64u, cursor = min(block, T.photons), end = min(block + 64u, T.photons);
   int read = 0;  // photons without a replay
   while (cursor < end) {
     unsigned gi = 0;
@@ -1480,6 +1514,13 @@ __global__ void __launch_bounds__(TAPE_BLOCK) tape_adjoint_kernel(Args a, AdjArg
         if (leave) head.z = 0u;
       }
       cursor = min(cursor + (unsigned)__popcll(mask), end);
+      if (cursor == end) {
+        block += waves * 64u;
+        if (block < T.photons) {
+          cursor = block;
+          end = min(block + 64u, T.photons);
+        }
+      }
       const unsigned long long lm = __ballot(leave);
       if (leave) left[n_left + lanes_below(lm)] = gi;
       n_left += __popcll(lm);
