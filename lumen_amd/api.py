@@ -376,13 +376,14 @@ class Engine:
         tape.held = held
         return tape
 
-    def upload(self, values: np.ndarray):
+    def upload(self, values: np.ndarray, current=None):
         """Return the packed values on the device, the previous upload again when they are the same.  The host does not
         wait for the copy, so another stream than the one that made it does, and the values are kept from reuse while
-        that stream may read them."""  # noqa: D205, D209
+        that stream may read them.  ``current``: the current stream, where the caller has it at hand."""  # noqa: D205, D209
         import torch
 
-        current = torch.cuda.current_stream(self.device)
+        if current is None:
+            current = torch.cuda.current_stream(self.device)
         last = self._uploads.get(values.nbytes)
         if last is not None and np.array_equal(last[0], values):
             _, t, stream, copied = last
@@ -540,7 +541,8 @@ def simulate(det, source, params: Params | None = None, *, samples: int | None =
     pk = packing.pack(det, p, edge_rows=edge_rows)
     if not np.array_equal(pk.layout, eng.layout):
         raise ValueError("simulate: these values change the detector's structure (a table's knot count)")
-    values = eng.upload(pk.values)
+    current = torch.cuda.current_stream(eng.device)
+    values = eng.upload(pk.values, current)
     ref_values = None
     if reference is not None:
         pr = packing.pack(det, reference, edge_rows=edge_rows)
@@ -556,7 +558,6 @@ def simulate(det, source, params: Params | None = None, *, samples: int | None =
     buf = torch.zeros((n_ev, max(eng.stride, 1)), dtype=torch.float64, device=eng.device)
     tally = buf[:, :eng.stride]
     health = torch.zeros(_lib.HEALTH_N, dtype=torch.float64, device=eng.device)
-    current = torch.cuda.current_stream(eng.device)
     st = current if stream is None else stream
     if st != current:  # the buffers' fills and the values' uploads (on the current stream) before the kernel
         st.wait_stream(current)
