@@ -37,6 +37,8 @@ def free(monkeypatch):
 
     base = sum(h.nbytes for h in api._TAPES)
     size = types.SimpleNamespace(free=0)
+    monkeypatch.setattr(api, "FREE_AGE", 0.0)
+    monkeypatch.setattr(api, "_FREE", {})
     monkeypatch.setattr(torch.cuda, "mem_get_info",
                         lambda d=None: (size.free + base - sum(h.nbytes for h in api._TAPES), 0))
     return size
@@ -63,6 +65,27 @@ def test_tapes_take_their_part(monkeypatch, free):
     got.clear()
     gc.collect()
     assert a.tape(ctl, False, n, False) is None  # one tape of more than its part
+
+
+def test_free_memory_is_looked_up_again(monkeypatch, free):
+    import torch
+
+    looks = []
+    real = torch.cuda.mem_get_info
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: looks.append(d) or real(d))
+    monkeypatch.setattr(_lib, "lib", lambda: _Sized())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(api, "FREE_AGE", 5.0)
+    now = [100.0]
+    monkeypatch.setattr(api.time, "monotonic", lambda: now[0])
+    gc.collect()
+    free.free = 10 * api.TAPE_PARTS
+    eng, ctl = _engine(), Controls().struct()
+    kept = [eng.tape(ctl, False, 4, False) for _ in range(3)]
+    assert [t is not None for t in kept] == [True, True, False] and looks == [0]  # the tapes since are counted
+    now[0] += 5.0
+    free.free = 12 * api.TAPE_PARTS
+    assert eng.tape(ctl, False, 4, False) is not None and looks == [0, 0]
 
 
 @pytest.mark.gpu
