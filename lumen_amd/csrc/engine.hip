@@ -1213,7 +1213,7 @@ __device__ inline Args stage_tables(const Args &a0) {
 // How a launch's photons are handed out (Range).  An explicit chunk is every block's size.  Else each wavefront has up to
 // OWN_PHOTONS of its own, in blocks of at most 64, and the work queue hands out the rest in small chunks.  Measured in the
 // tank, the kernel: 2^17 photons, all of them own, 0.14 ms, 0.28 in chunks of 256 that fill a sixth of the wavefronts;
-// 2^20 0.43 against 0.48; 2^22 1.26 against 1.36; 2^24 4.63 against 4.65.  Chunks of 64 to 128: below, the claims (12 ns
+// 2^20 0.42 against 0.48; 2^22 1.26 against 1.36; 2^24 4.61 against 4.65.  Chunks of 64 to 128: below, the claims (12 ns
 // each, one address) show on cheap photons.
 // Paths differ from source to source, so no wavefront may be left with many photons of one: its own blocks lie a stride of
 // all wavefronts apart, and 256 photons are what a queue of usual chunks would give it at once.  64 sources of which
@@ -1278,7 +1278,10 @@ __device__ __forceinline__ bool next_range(const Args &a, Range &r, int lane) {
   while (a.dyn_at < a.total) {
     unsigned long long c = 0;
     if (lane == 0) c = atomicAdd(a.queue, 1ull);
-    c = __shfl(c, 0);
+    // lane 0's as a number of the wavefront's, not of each lane's: four vector registers through every step (the tank with
+    // reference values, 2^22 photons: 1.445 ms from a shuffle, 1.405 so)
+    c = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(c >> 32)) << 32 |
+        (unsigned)__builtin_amdgcn_readfirstlane((int)c);
     const long long row = (long long)(c >> QUEUE_PARTS_LOG);
     if (row >= a.rows) break;
     const long long part = (long long)(c & (QUEUE_PARTS - 1));
