@@ -76,7 +76,8 @@ def _trace(run: _Run, values, tape=None):
 
 def adjoint(run: _Run, values, cot, tape=None):
     """Return the gradient slots (n_grad,) float64 of the loss whose cotangent on the tallies is ``cot``; ``tape``:
-    of these photons' paths (None: they are replayed)."""  # noqa: D205, D209
+    of these photons' paths (None: they are replayed).  ``run.adj_health`` counts every photon once; from a tape, its other
+    cells are those of the photons it replayed."""  # noqa: D205, D209
     import torch
 
     eng = run.eng

@@ -51,6 +51,7 @@ class BatchRun:
         self.health = torch.zeros(_lib.HEALTH_N, dtype=torch.float64, device=dev)
         self.cot = torch.zeros_like(self.tally)
         self.grad = torch.zeros(self.n_grad, dtype=torch.float64, device=dev)
+        # the adjoint's: every photon is counted once; from a tape, the other cells are those of the photons it replayed
         self.adj_health = torch.zeros_like(self.health)
         self.graph = graph
         self.tune = tune and controls is None

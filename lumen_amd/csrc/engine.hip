@@ -1220,10 +1220,12 @@ __device__ inline Args stage_tables(const Args &a0) {
 // every eighth has long paths (a sphere, 270 vertices against 1), 2^22 photons: 9.7 ms, 39.6 with three quarters of the
 // launch in equal shares of consecutive photons, 13.7 in chunks of 256.  The queue deals its chunks out of QUEUE_PARTS
 // parts of the launch in turn: taken in order, every wavefront would be at one source's photons at a time, and where the
-// events' tallies are in memory at one event's cells (256 sources in the tank, 5.4e7 photons: 16.8 ms in order, 15.5 so).
+// events' tallies are in memory at one event's cells (256 sources in the tank, 5.4e7 photons: 16.8 ms in order, 15.5 in 2
+// parts, 15.2 in 8 to 64; the argon box's replay of 2^24 photons, which ends with its longest photons, takes 1 % more in 8
+// parts than in order, 2 % in 64).
 constexpr long long OWN_PHOTONS = 256;
 constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
-constexpr int QUEUE_PARTS_LOG = 6, QUEUE_PARTS = 1 << QUEUE_PARTS_LOG;
+constexpr int QUEUE_PARTS_LOG = 3, QUEUE_PARTS = 1 << QUEUE_PARTS_LOG;
 
 // the split of the launch's photons over `waves` wavefronts (`given`: in chunks of the controls' size)
 __host__ __device__ inline void split_photons(Args &a, long long waves, bool given) {
@@ -2432,10 +2434,6 @@ static unsigned features_of(lh_model m, const Args &a, bool adj) {
   X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20) \
       X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31) X(32) X(33) X(34) X(35) X(36) X(37) X(38)  \
       X(39) X(40) X(41) X(42) X(43) X(44) X(45) X(46) X(47) X(64) X(66) X(72) X(74) X(192) X(194) X(200) X(202)
-
-
-
-
 
 // the workgroup size of a launch's kernel
 static int block_for(bool /* adjoint or forward */, unsigned /* features */) { return BLOCK; }

@@ -264,7 +264,8 @@ __device__ __forceinline__ float div_fast(float a, float b) {
 }
 
 // the correctly rounded quotient, where the source asks for it and not where the optimiser moves a division to: the
-// hardware's scaled Newton steps, the residual of the quotient applied twice
+// hardware's scaled Newton steps in the order its div_scale, div_fmas and div_fixup instructions are made for, the residual
+// of the quotient applied twice
 __device__ __forceinline__ float div_ieee(float a, float b) {
   bool sn, sd;
   const float n = __builtin_amdgcn_div_scalef(a, b, true, &sn), d = __builtin_amdgcn_div_scalef(a, b, false, &sd);
