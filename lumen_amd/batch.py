@@ -125,10 +125,14 @@ class BatchRun:
     def _choose_tape(self):
         """Set the tape of this run's forward and adjoint (None: it takes none), anew where its controls were replaced
         since.  A tape holds the forward's paths: the adjoint's controls are to ask for the same ones."""  # noqa: D205, D209
+        import torch
+
         shape = dict(chunk=0, blocks_per_cu=0, tally_global=False, nodes_global=False)
         paths = tuple(c._replace(**shape) for c in (self.controls, self.adj_controls or Controls()))
         if self._tape_of == paths:
             return
+        if self._tape is not None:  # a replay may still read it, on whatever stream it was started
+            torch.cuda.synchronize(self.eng.device)
         self._tape_of, self._tape, self._g_both = paths, None, None  # a captured graph holds the tape's address
         if paths[0] == paths[1]:
             ctl = self.controls.struct()

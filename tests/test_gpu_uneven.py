@@ -58,3 +58,27 @@ def test_long_paths_side_by_side(gpu, where, what):
     # the same deposits (terms) in FP64 sums of another order: n roundings of 1.1e-16 at most
     np.testing.assert_allclose(a, b, rtol=N * 1.2e-16, atol=N * 1.2e-16 * np.abs(b).max())
     assert own <= 1.25 * chunks
+
+
+WAVES = 256 * 12  # wavefronts of a launch on 256 CUs
+OWN = 256 * WAVES  # the photons that wavefronts have of their own; past them 8 parts of the queue, chunks of 64
+
+
+@pytest.mark.parametrize("n,chunk", [(64 * WAVES, 0), (64 * WAVES + 1, 0), (OWN - 1, 0), (OWN, 0), (OWN + 1, 0),
+                                     (OWN + 64, 0), (OWN + 8 * 64, 0), (OWN + 8 * 64 + 1, 0), (OWN + 33 * 64 + 5, 0),
+                                     (5000, 1), (WAVES * 7 + 1, 7), (WAVES * 7 + 8 * 7 + 1, 7), (100_003, 1 << 17)])
+def test_every_photon_once_at_the_edges_of_the_split(gpu, n, chunk):
+    """The last own block, the queue's first chunk, a part that is one chunk short, chunks of 1 and of more than all."""
+    import lumen_amd as L
+    from lumen_amd.detector import example_tank
+
+    det = example_tank()
+    src = L.sources.Point((0.05, 0.0, 0.1), lam=400.0, n_photons=2e5)
+    a = L.simulate(det, src, samples=n, seed=4, controls=Controls(chunk=chunk))
+    b = L.simulate(det, src, samples=n, seed=4, chunk=50_000)  # launches of photons that are all own
+    for k in ("photons", "vertices", "records"):
+        assert getattr(a.health, k) == getattr(b.health, k)
+    assert a.health.photons == n
+    # the same deposits in FP64 sums of another order: n roundings of 1.1e-16 at most
+    for x, y in ((a.arrivals, b.arrivals), (a.charge, b.charge), (a.arrival2, b.arrival2)):
+        np.testing.assert_allclose(x.cpu().numpy(), y.cpu().numpy(), rtol=n * 1.2e-16, atol=0.0)
