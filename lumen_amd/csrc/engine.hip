@@ -85,6 +85,15 @@ struct LayoutAt {
   int media, class_medium, row_of, rows, classes;
 };
 
+// how a launch's photons are handed out to its wavefronts (split_photons)
+struct Split {
+  long long total;
+  long long block, stride;  // each wavefront's own blocks of photons: their size, the step from one to its next
+  long long dyn_at, rows;   // where the own blocks end: the work queue hands out the photons past it, in QUEUE_PARTS
+                            // parts of `rows` chunks each
+  long long chunk;          // the photons a wavefront takes from the queue at once
+};
+
 struct Args {
   Geo g;
   const int *__restrict__ L;
@@ -99,9 +108,7 @@ struct Args {
   uint32_t k0, k1;
   float roulette, max_dist, reach;
   int max_vert, chunk;
-  long long block, stride;  // each wavefront's own blocks of photons: their size, the step from one to its next (Range)
-  long long dyn_at, rows;   // where the own blocks end: the work queue hands out the photons past it, in QUEUE_PARTS
-                            // parts of `rows` chunks each
+  Split split;
   int keep_zero;  // 1: a photon whose live weight became 0 walks on (the reference's records); 0: it ends
   int reach_on;   // 1: the reach bound where the model has one (the controls' reach_bound)
   double *__restrict__ tally;
@@ -1221,35 +1228,51 @@ __device__ inline Args stage_tables(const Args &a0) {
 // launch in equal shares of consecutive photons, 13.7 in chunks of 256.  The queue deals its chunks out of QUEUE_PARTS
 // parts of the launch in turn: taken in order, every wavefront would be at one source's photons at a time, and where the
 // events' tallies are in memory at one event's cells (256 sources in the tank, 5.4e7 photons: 16.8 ms in order, 15.5 in 2
-// parts, 15.2 in 8 to 64; the argon box's replay of 2^24 photons, which ends with its longest photons, takes 1 % more in 8
+// parts, 15.2 in 8 to 64; the argon box's replay of 2^24 photons, which ends with its longest photons, took 1 % more in 8
 // parts than in order, 2 % in 64).
 constexpr long long OWN_PHOTONS = 256;
 constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
 constexpr int QUEUE_PARTS_LOG = 3, QUEUE_PARTS = 1 << QUEUE_PARTS_LOG;
 
-// the split of the launch's photons over `waves` wavefronts (`given`: in chunks of the controls' size)
-__host__ __device__ inline void split_photons(Args &a, long long waves, bool given) {
+// the split of `total` photons over `waves` wavefronts (`chunk` > 0: in chunks of that many)
+__host__ __device__ inline Split split_photons(long long total, long long waves, long long chunk) {
+  Split s{total, chunk, 0, 0, 0, chunk};
   long long count = 1;  // own blocks
-  a.block = a.chunk;
-  if (!given) {
-    const long long share = (a.total + waves - 1) / waves, some = share / 16;
+  if (chunk <= 0) {
+    const long long share = (total + waves - 1) / waves, some = share / 16;
     const long long own = share < OWN_PHOTONS ? share : OWN_PHOTONS;
-    a.chunk = (int)(some < MIN_CHUNK ? MIN_CHUNK : some > MAX_CHUNK ? MAX_CHUNK : some);
+    s.chunk = some < MIN_CHUNK ? MIN_CHUNK : some > MAX_CHUNK ? MAX_CHUNK : some;
     count = (own + MIN_CHUNK - 1) / MIN_CHUNK;
-    a.block = own > 0 ? (own + count - 1) / count : 0;
+    s.block = own > 0 ? (own + count - 1) / count : 0;
   }
-  a.stride = waves * a.block;
-  a.dyn_at = a.total < a.stride * count ? a.total : a.stride * count;
-  const long long row = (long long)QUEUE_PARTS * a.chunk;
-  a.rows = (a.total - a.dyn_at + row - 1) / row;
+  s.stride = waves * s.block;
+  s.dyn_at = total < s.stride * count ? total : s.stride * count;
+  const long long row = QUEUE_PARTS * s.chunk;
+  s.rows = (total - s.dyn_at + row - 1) / row;
+  return s;
 }
 
-// ... of the photons a tape left to the replay, their number known on the device alone.  The queue matters here too: with an
-// equal share for every wavefront the launch waits for the one that got the longest paths (a sphere with facets, R 0.99,
-// 2^22 photons, three quarters of them replayed: adjoint 137 ms, 110 with the queue)
-__device__ __forceinline__ void split_replay(Args &a) {
-  a.total = (long long)(unsigned)__builtin_amdgcn_readfirstlane((int)a.replay[0]);
-  split_photons(a, (long long)gridDim.x * (blockDim.x >> 6), a.chunk > 0);
+// the kernel's first argument, read anew at each call: the barrier keeps the compiler from loading a field at the kernel's
+// start and holding it in scalar registers through every step
+typedef const __attribute__((address_space(4))) Args KernelArgs;
+__device__ __forceinline__ KernelArgs *kernel_args() {
+  KernelArgs *a = (KernelArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+// this launch's split, wanted where a range ends.  Its twelve words held through the step push others to scratch (argon box,
+// 2^15 photons, the longest photon's chain: 95.8 ms so held, 92.7 read anew).  In the adjoint, of the photons that a tape
+// left to the replay: their number is known on the device alone.  The queue matters there too: with an equal share for
+// every wavefront the launch waits for the one that got the longest paths (a sphere with facets, R 0.99, 2^22 photons,
+// three quarters of them replayed: adjoint 137 ms, 110 with the queue)
+template <bool ADJ>
+__device__ __forceinline__ Split launch_split() {
+  KernelArgs *a = kernel_args();
+  if (ADJ && a->replay)
+    return split_photons((unsigned)__builtin_amdgcn_readfirstlane((int)a->replay[0]),
+                         (long long)gridDim.x * (blockDim.x >> 6), a->chunk);
+  return Split{a->split.total, a->split.block, a->split.stride, a->split.dyn_at, a->split.rows, a->split.chunk};
 }
 
 // A wavefront's range of the launch's photons.  Its first blocks are its own by its index, wavefront w of every workgroup
@@ -1261,36 +1284,40 @@ struct Range {
   bool drained;
 };
 
-__device__ __forceinline__ Range first_range(const Args &a) {
+template <bool ADJ>
+__device__ __forceinline__ Range first_range() {
+  const Split s = launch_split<ADJ>();
   const long long w = (long long)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-  const long long b = w * a.block;
-  return Range{min(b, a.dyn_at), min(b + a.block, a.dyn_at), false};
+  const long long b = w * s.block;
+  return Range{min(b, s.dyn_at), min(b + s.block, s.dyn_at), false};
 }
 
 // the next block or chunk when the range is used up: false once there is none.  The next own block lies a stride past the
-// one that ends; only the launch's last is cut short, at dyn_at.  The parts are equal but for the last, which may hold fewer
-// chunks than it has numbers
-__device__ __forceinline__ bool next_range(const Args &a, Range &r, int lane) {
-  const long long next = r.end - a.block + a.stride;
-  if (r.end < a.dyn_at && next < a.dyn_at) {
+// one that ends; only the launch's last is cut short, at dyn_at.  The last parts may hold fewer chunks than they have
+// numbers
+template <bool ADJ>
+__device__ __forceinline__ bool next_range(Range &r, int lane) {
+  const Split s = launch_split<ADJ>();
+  const long long next = r.end - s.block + s.stride;
+  if (r.end < s.dyn_at && next < s.dyn_at) {
     r.cursor = next;
-    r.end = min(next + a.block, a.dyn_at);
+    r.end = min(next + s.block, s.dyn_at);
     return true;
   }
-  while (a.dyn_at < a.total) {
+  unsigned long long *queue = kernel_args()->queue;
+  while (s.dyn_at < s.total) {
     unsigned long long c = 0;
-    if (lane == 0) c = atomicAdd(a.queue, 1ull);
+    if (lane == 0) c = atomicAdd(queue, 1ull);
     // lane 0's as a number of the wavefront's, not of each lane's: four vector registers through every step (the tank with
     // reference values, 2^22 photons: 1.445 ms from a shuffle, 1.405 so)
     c = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(c >> 32)) << 32 |
         (unsigned)__builtin_amdgcn_readfirstlane((int)c);
-    const long long row = (long long)(c >> QUEUE_PARTS_LOG);
-    if (row >= a.rows) break;
-    const long long part = (long long)(c & (QUEUE_PARTS - 1));
-    const long long base = a.dyn_at + (part * a.rows + row) * a.chunk;
-    if (base < a.total) {
+    const long long row = (long long)(c >> QUEUE_PARTS_LOG), part = (long long)(c & (QUEUE_PARTS - 1));
+    if (row >= s.rows) break;
+    const long long base = s.dyn_at + (part * s.rows + row) * s.chunk;
+    if (base < s.total) {
       r.cursor = base;
-      r.end = min(base + a.chunk, a.total);
+      r.end = min(base + s.chunk, s.total);
       return true;
     }
   }
@@ -1313,7 +1340,7 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
   Acc acc{};
   bool alive = false;
   const int lane = threadIdx.x & 63;
-  Range r = first_range(a);
+  Range r = first_range<false>();
   for (;;) {
     // refill the lanes whose photon ended from the wavefront's chunk of the work queue
     bool need = !alive, taken = false;
@@ -1322,7 +1349,7 @@ __global__ void __launch_bounds__(block_of<F>()) LH_OCC_FWD(F) trace_kernel(Args
     while (mask != 0ull && !r.drained) {
       const long long avail = r.end - r.cursor;
       if (avail <= 0) {
-        if (!next_range(a, r, lane)) break;
+        if (!next_range<false>(r, lane)) break;
         continue;
       }
       const int rank = lanes_below(mask);
@@ -1379,14 +1406,13 @@ __global__ void __launch_bounds__(adj_block_of<F>())
   for (int i = threadIdx.x; i < b.n_grad; i += blockDim.x) sg[i] = 0.0;
   clear_block_cells();
   stage_nodes(a0.g);
-  Args a = stage_tables<F>(a0);
-  if (a.replay) split_replay(a);
+  const Args a = stage_tables<F>(a0);
   __syncthreads();
   Photon p;
   Acc acc{};
   bool alive = false;
   const int lane = threadIdx.x & 63;
-  Range r = first_range(a);
+  Range r = first_range<true>();
   for (;;) {
     bool need = !alive, taken = false;
     long long gi = 0;
@@ -1394,7 +1420,7 @@ __global__ void __launch_bounds__(adj_block_of<F>())
     while (mask != 0ull && !r.drained) {
       const long long avail = r.end - r.cursor;
       if (avail <= 0) {
-        if (!next_range(a, r, lane)) break;
+        if (!next_range<true>(r, lane)) break;
         continue;
       }
       const int rank = lanes_below(mask);
@@ -2543,10 +2569,10 @@ static size_t place_lds(lh_model m, Args &a, const void *fn, int block, size_t c
   return end;
 }
 
-static void claim_schedule(Args &a, const lh_controls *ctl, int grid, int block, hipStream_t st) {
+static void claim_schedule(Args &a, int grid, int block, hipStream_t st) {
   if (a.replay) return;  // split on the device, its queue cleared before the reader
-  split_photons(a, (long long)grid * (block / 64), ctl && ctl->chunk > 0);
-  if (a.dyn_at < a.total || a.tape.cells)
+  a.split = split_photons(a.total, (long long)grid * (block / 64), a.chunk);
+  if (a.split.dyn_at < a.total || a.tape.cells)
     hipLaunchKernelGGL(reset_queue, dim3(1), dim3(1), 0, st, a.queue, a.tape.cells ? &a.tape.cells[0].x : nullptr);
 }
 
@@ -2564,7 +2590,7 @@ static void launch_adjoint(lh_model m, Args &a, const AdjArgs &b, const lh_contr
   m->last_launch[1] = grid / std::max(m->cus, 1);
   m->last_launch[2] = (int32_t)bytes;
   m->last_launch[7] = (int32_t)f | 0x100;
-  claim_schedule(a, ctl, grid, block_for(true, f), st);
+  claim_schedule(a, grid, block_for(true, f), st);
   launch_kernel(true, f, dim3(grid), bytes, st, a, b, 0);
 }
 
@@ -2584,7 +2610,7 @@ static void launch_trace(lh_model m, Args &a, int n_events, const lh_controls *c
   m->last_launch[1] = grid / std::max(m->cus, 1);
   m->last_launch[2] = (int32_t)bytes;
   m->last_launch[7] = (int32_t)fk;
-  claim_schedule(a, ctl, grid, block_for(false, fk), st);
+  claim_schedule(a, grid, block_for(false, fk), st);
   launch_kernel(false, fk, dim3(grid), bytes, st, a, AdjArgs{}, n_lds);
 }
 
