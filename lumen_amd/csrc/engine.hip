@@ -1220,15 +1220,15 @@ __device__ inline Args stage_tables(const Args &a0) {
 // How a launch's photons are handed out (Range).  An explicit chunk is every block's size.  Else each wavefront has up to
 // OWN_PHOTONS of its own, in blocks of at most 64, and the work queue hands out the rest in small chunks.  Measured in the
 // tank, the kernel: 2^17 photons, all of them own, 0.14 ms, 0.28 in chunks of 256 that fill a sixth of the wavefronts;
-// 2^20 0.42 against 0.48; 2^22 1.26 against 1.36; 2^24 4.61 against 4.65.  Chunks of 64 to 128: below, the claims (12 ns
+// 2^20 0.41 against 0.48; 2^22 1.25 against 1.36; 2^24 4.60 against 4.64.  Chunks of 64 to 128: below, the claims (12 ns
 // each, one address) show on cheap photons.
 // Paths differ from source to source, so no wavefront may be left with many photons of one: its own blocks lie a stride of
 // all wavefronts apart, and 256 photons are what a queue of usual chunks would give it at once.  64 sources of which
-// every eighth has long paths (a sphere, 270 vertices against 1), 2^22 photons: 9.7 ms, 39.6 with three quarters of the
+// every eighth has long paths (a sphere, 270 vertices against 1), 2^22 photons: 9.0 ms, 39.3 with three quarters of the
 // launch in equal shares of consecutive photons, 13.7 in chunks of 256.  The queue deals its chunks out of QUEUE_PARTS
 // parts of the launch in turn: taken in order, every wavefront would be at one source's photons at a time, and where the
-// events' tallies are in memory at one event's cells (256 sources in the tank, 5.4e7 photons: 16.8 ms in order, 15.5 in 2
-// parts, 15.2 in 8 to 64; the argon box's replay of 2^24 photons, which ends with its longest photons, took 1 % more in 8
+// events' tallies are in memory at one event's cells (256 sources in the tank, 5.4e7 photons: 16.8 ms in order, 15.4 in 2
+// parts, 15.1 in 8; the argon box's replay of 2^24 photons, which ends with its longest photons, took 1 % more in 8
 // parts than in order, 2 % in 64).
 constexpr long long OWN_PHOTONS = 256;
 constexpr long long MIN_CHUNK = 64, MAX_CHUNK = 128;
